@@ -20,6 +20,7 @@ hipError_t grad_impl(const GridOpArgs& ga, const void* G, const void* P, void* g
   o.val = static_cast<cplx<T>*>(gval);
   o.P = static_cast<const cplx<T>*>(P);
   for (int d = 0; d < 3; ++d) o.gcoord[d] = d < D ? static_cast<T*>(gcoord[d]) : nullptr;
+  o.store = ga.n_trans == 1;
   return dispatch_ns(ga.g->ns, [&](auto nsc) -> hipError_t {
     constexpr int NS = decltype(nsc)::value;
     if (tiled) {
@@ -64,6 +65,12 @@ hipError_t grad_dim(const GridOpArgs& ga, const void* G, const void* P, void* gv
 hipError_t launch_interp_grad(const GridOpArgs& ga, const void* G, const void* P, void* gval, void* const gcoord[3],
                               hipStream_t s) {
   if (ga.ps->M == 0) return hipSuccess;
+  if (ga.n_trans > 1)
+    for (int d = 0; d < ga.g->dim; ++d)
+      if (gcoord[d]) {
+        hipError_t e = launch_zero(gcoord[d], ga.ps->M * (ga.prec == kF32 ? 4 : 8), s);
+        if (e != hipSuccess) return e;
+      }
   if (ga.prec == kF32) {
     return ga.ps->coord_f64 ? grad_dim<float, double>(ga, G, P, gval, gcoord, s)
                             : grad_dim<float, float>(ga, G, P, gval, gcoord, s);

@@ -215,7 +215,8 @@ hipError_t launch_interp_many(const GridOpArgs* a, int count, const void* const*
 // Fused gather with kernel-derivative weights.  For each point i and transform t:
 //   S0 = sum G w, S_ax = sum G dW/d ax   (dW/d ax includes the -nf/2pi chain factor)
 //   gval[t][i] = S0                               (if gval != nullptr)
-//   gcoord_ax[i] += Re(conj(P[t][i]) * S_ax)      (if gcoord[ax] != nullptr; zeroed by caller)
+//   gcoord_ax[i] = sum_t Re(conj(P[t][i]) * S_ax) (if gcoord[ax] != nullptr)
+// One transform stores each point's gradient; several add into arrays that it clears first.
 hipError_t launch_interp_grad(const GridOpArgs& a, const void* G, const void* P, void* gval, void* const gcoord[3],
                               hipStream_t s);
 

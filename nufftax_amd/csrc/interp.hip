@@ -19,6 +19,7 @@ hipError_t interp_impl(const GridOpArgs& ga, const void* fw, void* c, hipStream_
   o.val = static_cast<cplx<T>*>(c);
   o.P = nullptr;
   o.gcoord[0] = o.gcoord[1] = o.gcoord[2] = nullptr;
+  o.store = false;
   return dispatch_ns(ga.g->ns, [&](auto nsc) -> hipError_t {
     constexpr int NS = decltype(nsc)::value;
     if (tiled) {

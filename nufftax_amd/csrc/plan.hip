@@ -874,10 +874,7 @@ int nufftx_vjp(nufftx_plan p, const void* src, const void* g, void* grad_src, vo
   if (!g) return fail(NUFFTX_ERR_INVALID_ARG, "null cotangent");
   void* gc[3] = {gx, p->dim > 1 ? gy : nullptr, p->dim > 2 ? gz : nullptr};
   const bool want_coord = gc[0] || gc[1] || gc[2];
-  const size_t rsz = p->prec == kF32 ? 4 : 8;
   if (want_coord && !src) return fail(NUFFTX_ERR_INVALID_ARG, "coordinate gradients need the primal input");
-  for (int d = 0; d < 3; ++d)
-    if (gc[d]) LAUNCH(launch_zero(gc[d], p->M * (int64_t)rsz, p->stream));
   const int s = -p->isign;
   if (p->type == 1) {
     // G = FFT_{-isign}(pad(g / phihat)) -- adjoint of deconvolve-shuffle and FFT
@@ -938,9 +935,6 @@ int nufftx_gather_grad(nufftx_plan p, const void* G, const void* P, void* gval, 
   void* gc[3] = {gx, p->dim > 1 ? gy : nullptr, p->dim > 2 ? gz : nullptr};
   const bool want_coord = gc[0] || gc[1] || gc[2];
   if (!G || (want_coord && !P)) return fail(NUFFTX_ERR_INVALID_ARG, "null data pointer");
-  const size_t rsz = p->prec == kF32 ? 4 : 8;
-  for (int d = 0; d < 3; ++d)
-    if (gc[d]) LAUNCH(launch_zero(gc[d], p->M * (int64_t)rsz, p->stream));
   if (want_coord) {
     LAUNCH(launch_interp_grad(gop(p, p->ps, p->g), G, P, gval, gc, p->stream));
   } else if (gval) {

@@ -748,7 +748,8 @@ template <typename T, int D, bool DERIV>
 struct GatherOut {
   cplx<T>* val;           // [n_trans][M] or nullptr
   const cplx<T>* P;       // [n_trans][M] pointwise factor for coordinate gradients
-  T* gcoord[3];           // [M] each, accumulated, or nullptr
+  T* gcoord[3];           // [M] each, or nullptr: added to (zeroed by the caller), or stored
+  bool store;             // one transform: the point's only gradient is stored, not added
 };
 
 template <typename T, int D, bool DERIV>
@@ -763,7 +764,12 @@ __device__ __forceinline__ void emit_point(const SIArgs<T>& a, const GatherOut<T
       if (o.gcoord[d]) {
         // Re(conj(P) * S) with the dz/dx chain factor
         const T g = (pv.re * sd[d].re + pv.im * sd[d].im) * a.dscale[d];
-        atomic_add_global(o.gcoord[d] + p, g);
+        // random global FP32 atomics run at ~18 G/s on MI355X, and two of them per point took most
+        // of the 111 us of this gather over 1M points (2D, ns = 8; the value gather takes 27)
+        if (o.store)
+          o.gcoord[d][p] = g;
+        else
+          atomic_add_global(o.gcoord[d] + p, g);
       }
     }
   }
@@ -1035,6 +1041,7 @@ __global__ void __launch_bounds__(256) k_gather_tiled_many(GatherMany m) {
   o.val = m.out[p];
   o.P = nullptr;
   o.gcoord[0] = o.gcoord[1] = o.gcoord[2] = nullptr;
+  o.store = false;
   gather_tiled_block<float, CT, D, NS, false, REC>(m.a[p], m.fw[p], o, (int)blockIdx.x - m.first[p],
                                                    (int)blockIdx.y);
 }

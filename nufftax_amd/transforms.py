@@ -213,16 +213,20 @@ def _vjp_type12(kind, meta: _Meta, src, coords, g, need_src, need_coord):
     else:
         gg = g.reshape(n_trans, M).to(cdt).contiguous()
     grad_src = torch.empty_like(ss) if need_src else None
-    gcoord = [torch.zeros(M, dtype=rdt, device=dev) if need_coord[d] else None for d in range(dim)]
+    # one chunk writes the gradients themselves; several (more than MAX_TRANS transforms) add up
+    one = 1 <= n_trans <= MAX_TRANS
+    new = torch.empty if one else torch.zeros
+    gcoord = [new(M, dtype=rdt, device=dev) if need_coord[d] else None for d in range(dim)]
     for s, e in _chunks(n_trans):
         plan = transform_plan(kind, dim, n_modes, e - s, meta.eps, meta.isign, meta.upsampfac_T, prec, dev)
-        part = [torch.empty(M, dtype=rdt, device=dev) if gc is not None else None for gc in gcoord]
+        part = gcoord if one else [torch.empty_like(gc) if gc is not None else None for gc in gcoord]
         with plan.lock:
             plan.setpts(xs)
             plan.vjp(ss[s:e], gg[s:e], grad_src[s:e] if grad_src is not None else None, part)
-        for d in range(dim):
-            if gcoord[d] is not None:
-                gcoord[d] += part[d]
+        if not one:
+            for gc, pc in zip(gcoord, part):
+                if gc is not None:
+                    gc += pc
     if grad_src is not None:
         grad_src = grad_src.reshape(src.shape).to(src.dtype)
     out_coords = [gc.to(coords[d].dtype) if gc is not None else None for d, gc in enumerate(gcoord)]

@@ -264,3 +264,31 @@ def test_c64_coordinate_grads_wide_reads_match(rng, dim, nm, kind, monkeypatch):
     b = grads("0")
     for u, v in zip(a, b):
         assert R.rel_l2(u, v) < 1e-5
+
+
+@pytest.mark.parametrize("dim,M,n_trans,double", [(1, 1, 1, False), (2, 257, 1, False), (2, 257, 3, False),
+                                                  (3, 2500, 1, False), (3, 2500, 2, True), (1, 1030, 1, True)])
+def test_plan_vjp_writes_whole_gradients(rng, dim, M, n_trans, double):
+    """The gradient arrays of nufftx_vjp need no clearing, for one transform (stored) and for
+    several (added up): NaN before, the direct sums' gradients after.  Tolerance: eps 1e-6 (FP32)
+    or 1e-9 (FP64) times the mode numbers' scale, an order of magnitude above it."""
+    from nufftax_amd._plan import F32, F64, Plan
+
+    nm = (14, 9, 6)[:dim]
+    rdt, cdt = (torch.float64, torch.complex128) if double else (torch.float32, torch.complex64)
+    eps = 1e-9 if double else 1e-6
+    xs = [_t(rng.uniform(-np.pi, np.pi, M), rdt) for _ in range(dim)]
+    c = rng.standard_normal((n_trans, M)) + 1j * rng.standard_normal((n_trans, M))
+    shape = (n_trans,) + tuple(reversed(nm))
+    g = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    plan = Plan.transform(1, dim, nm, n_trans, eps, 1, 2.0, F64 if double else F32, 0, torch.device(DEV, 0))
+    plan.setpts(xs)
+    grads = [torch.full((M,), float("nan"), dtype=rdt, device=DEV) for _ in range(dim)]
+    plan.vjp(_t(c, cdt), _t(g, cdt), None, grads)
+    xd = [_np(x).astype(np.float64) for x in xs]
+    ks = np.meshgrid(*[np.arange(-(n // 2), (n + 1) // 2) for n in reversed(nm)], indexing="ij")[::-1]
+    E = np.exp(1j * sum(k.ravel()[:, None] * x[None] for k, x in zip(ks, xd)))
+    cc, gg = _np(_t(c, cdt)).astype(complex), _np(_t(g, cdt)).astype(complex).reshape(n_trans, -1)
+    for d in range(dim):
+        want = np.real(np.einsum("tj,tk,kj,k->j", cc, gg.conj(), E, 1j * ks[d].ravel(), optimize=True))
+        assert R.rel_l2(_np(grads[d]), want) < 20 * eps
