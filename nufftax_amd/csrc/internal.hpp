@@ -76,6 +76,14 @@ struct PointSet {
   int64_t cap_slot = 0, cap_packed = 0, cap_cs = 0;
   int64_t cap_recs = 0, cap_sub_off = 0, cap_cmax = 0;
   int64_t cap_M = 0, cap_keys = 0, cap_hist = 0, cap_part = 0, cap_bins = 0, cap_sub = 0, cap_sub_start = 0;
+  // 3D FP64 point sets spread by output regions (spread64.hip), per execute
+  double* tab64 = nullptr;       // M * 3 ns kernel weights in sorted order
+  int4* start64 = nullptr;       // M support starts
+  double2* cs64 = nullptr;       // n_trans * M strengths in sorted order
+  int2* bad64 = nullptr;         // (slot, transform) pairs that are not finite
+  int4* task64 = nullptr;        // tasks: {region, first, last + 1 candidate, tasks of the region}
+  int32_t* heavy64 = nullptr;    // 4 counters, then the regions of several tasks
+  int64_t cap_tab64 = 0, cap_start64 = 0, cap_cs64 = 0, cap_bad64 = 0, cap_task64 = 0, cap_heavy64 = 0;
   std::vector<void*> retired;    // outgrown buffers, freed by pointset_free
 };
 
@@ -219,6 +227,12 @@ hipError_t launch_interp_many(const GridOpArgs* a, int count, const void* const*
 // One transform stores each point's gradient; several add into arrays that it clears first.
 hipError_t launch_interp_grad(const GridOpArgs& a, const void* G, const void* P, void* gval, void* const gcoord[3],
                               hipStream_t s);
+
+// ---- spread64.hip: 3D FP64 spreading by output regions
+constexpr int64_t kSpread64MinPoints = 2048;
+bool spread64_applicable(const Geometry& g, int prec, int64_t M);
+hipError_t spread64_reserve(PointSet& ps, const Geometry& g, int64_t n_trans);  // buffers for M points
+hipError_t launch_spread64(const GridOpArgs& a, const void* c, void* fw, hipStream_t s);
 
 // ---- elementwise.hip
 hipError_t launch_zero(void* p, int64_t bytes, hipStream_t s);

@@ -506,6 +506,8 @@ int sort_points(nufftx_plan p, PointSet& ps, const Geometry& g, bool interp, boo
     e = pointset_subsort(ps, g, p->stream);
     if (e != hipSuccess) return fail(NUFFTX_ERR_HIP, std::string("sub-bin sort: ") + hipGetErrorString(e));
   }
+  if (spread && spread64_applicable(g, p->prec, ps.M) && spread64_reserve(ps, g, p->n_trans) != hipSuccess)
+    return fail(NUFFTX_ERR_ALLOC, "FP64 spreading buffers");
   // the FP32 spreading kernels' strength bound (n_trans values and the per-block partial
   // maxima) is sized here, so that execute allocates nothing for a point set of this size
   if (p->prec == kF32) {

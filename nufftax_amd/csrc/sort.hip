@@ -825,7 +825,8 @@ hipError_t pointset_pack3d(PointSet& ps, const Geometry& g, const void* c, int64
 
 void pointset_free(PointSet& ps) {
   void* bufs[] = {ps.perm, ps.keys, ps.hist, ps.scan_part, ps.scan_sum, ps.bin_start, ps.sub_start, ps.subprob,
-                  ps.nsub, ps.recs, ps.crec, ps.sub_off, ps.cmax, ps.slot, ps.packed, ps.cs};
+                  ps.nsub, ps.recs, ps.crec, ps.sub_off, ps.cmax, ps.slot, ps.packed, ps.cs,
+                  ps.tab64, ps.start64, ps.cs64, ps.bad64, ps.task64, ps.heavy64};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   for (void* p : ps.retired) (void)hipFree(p);
@@ -843,6 +844,13 @@ void pointset_free(PointSet& ps) {
   ps.cs = nullptr;
   ps.has_slot = false;
   ps.cap_slot = ps.cap_packed = ps.cap_cs = 0;
+  ps.tab64 = nullptr;
+  ps.start64 = nullptr;
+  ps.cs64 = nullptr;
+  ps.bad64 = nullptr;
+  ps.task64 = nullptr;
+  ps.heavy64 = nullptr;
+  ps.cap_tab64 = ps.cap_start64 = ps.cap_cs64 = ps.cap_bad64 = ps.cap_task64 = ps.cap_heavy64 = 0;
   ps.has_recs = false;
   ps.recs_subbin = false;
   ps.cap_recs = ps.cap_sub_off = ps.cap_cmax = 0;

@@ -938,3 +938,74 @@ def test_fused_fft_matches_rocfft(rng, monkeypatch, nm, sigma, isign, modeord):
     fused, refs = run(False)
     rocfft, _ = run(True)
     _check_fused_vs_rocfft(fused, rocfft, refs or (None, None), sigma)
+
+
+# ------------------------------------------------------------------ 3D FP64 spread by output regions
+
+
+@pytest.mark.parametrize("nfs,ns,M,dist", [
+    ((16, 16, 16), 12, 2048, "uniform"),    # two regions
+    ((17, 33, 20), 12, 2049, "uniform"),    # remainders on every axis
+    ((80, 64, 64), 8, 3001, "uniform"),
+    ((28, 28, 28), 14, 2500, "uniform"),    # supports of half the grid; regions see every bin
+    ((16, 20, 18), 16, 2200, "uniform"),    # supports as long as an axis
+    ((70, 51, 44), 10, 6000, "uniform"),
+    ((48, 48, 40), 12, 9000, "spot"),       # regions of many tasks
+    ((64, 20, 33), 12, 5000, "edges"),      # starts on grid points and at the wrap
+])
+@pytest.mark.parametrize("add", [False, True])
+def test_spread64_regions(rng, nfs, ns, M, dist, add):
+    """FP64 accumulation in another order than the oracle's: 1e-13 of the grid's norm."""
+    from nufftax_amd._plan import F64, Plan
+
+    kp = R.compute_kernel_params({2: 1e-1, 4: 1e-3, 6: 1e-5, 8: 1e-7, 10: 1e-9, 12: 1e-11, 14: 1e-13, 16: 1e-15}[ns])
+    assert kp.nspread == ns
+    if dist == "uniform":
+        coords = [rng.uniform(-np.pi, np.pi, M) for _ in nfs]
+    elif dist == "spot":
+        coords = [np.concatenate([rng.normal(3.0, 0.05, M - 100), rng.uniform(-np.pi, np.pi, 100)]) for _ in nfs]
+    else:
+        coords = [rng.integers(0, n, M) * (2 * np.pi / n) - np.pi for n in nfs]
+        coords[0][:4] = [np.pi, -np.pi, np.nextafter(np.pi, 0), 0.0]
+    c = rng.standard_normal((2, M)) + 1j * rng.standard_normal((2, M))
+    plan = Plan.grid_op(3, nfs, ns, kp.beta, kp.c, 2, F64, torch.device(DEV, 0))
+    plan.setpts([_t(x) for x in coords])
+    shape = (2,) + tuple(reversed(nfs))
+    old = rng.standard_normal(shape) + 1j * rng.standard_normal(shape) if add else np.full(shape, np.nan + 0j)
+    fw = _t(old)
+    (plan.spread_add if add else plan.spread)(_t(c), fw)
+    got = _np(fw) - (old if add else 0.0)
+    if dist == "edges":
+        # a point on a grid point has its support's first or last cell, of weight exp(-beta), by the rounding of
+        # its fold, which is the library's own: the reference is the general path, which takes fewer than 2048 points
+        want = np.zeros(shape, complex)
+        for s in range(0, M, 2000):
+            plan.setpts([_t(x[s:s + 2000]) for x in coords])
+            plan.spread(_t(c[:, s:s + 2000]), fw)
+            want += _np(fw)
+    else:
+        want = [R.spread([R.wrap_pi(x) for x in coords], c[t], nfs, kp) for t in range(2)]
+    for t in range(2):
+        assert R.rel_l2(got[t], want[t]) < 1e-13
+
+
+def test_spread64_regions_non_finite(rng):
+    """A non-finite strength reaches the cells of its point's support and no others."""
+    from nufftax_amd._plan import F64, Plan
+
+    nfs, M = (40, 40, 24), 2100
+    kp = R.compute_kernel_params(1e-11)
+    coords = [rng.uniform(-np.pi, np.pi, M) for _ in nfs]
+    c = rng.standard_normal((2, M)) + 1j * rng.standard_normal((2, M))
+    plan = Plan.grid_op(3, nfs, kp.nspread, kp.beta, kp.c, 2, F64, torch.device(DEV, 0))
+    plan.setpts([_t(x) for x in coords])
+    shape = (2,) + tuple(reversed(nfs))
+    ref, got = _t(np.zeros(shape, complex)), _t(np.zeros(shape, complex))
+    plan.spread(_t(c), ref)
+    c[1, 7] = np.inf + 1j
+    plan.spread(_t(c), got)
+    ref, got = _np(ref), _np(got)
+    assert R.rel_l2(got[0], ref[0]) < 1e-13
+    touched = R.spread([R.wrap_pi(x)[7:8] for x in coords], np.ones(1, complex), nfs, kp) != 0
+    assert np.isposinf(got[1].real[touched]).all()
+    assert R.rel_l2(got[1][~touched], ref[1][~touched]) < 1e-13
