@@ -267,6 +267,23 @@ void fft2_plan_free(Fft2Plan& fp);
 hipError_t fft2_shuffle(Fft2Plan& fp, const DeconvArgs& a, const void* grid, void* f, int isign, hipStream_t s);
 hipError_t fft2_pad(Fft2Plan& fp, const DeconvArgs& a, const void* f, void* grid, int isign, hipStream_t s);
 
+// ---- fftn.hip: the same for 2-3-5-smooth grids, FP32 and FP64
+struct FftnPlan {
+  struct Axis {
+    int n = 1;
+    std::vector<int> radix;
+    void* tw = nullptr;  // n twiddles
+  } axis[3];             // 1D grids of two passes: their two lengths
+  int split = 0;         // 1D of two passes: the first length
+  void* mid = nullptr;   // one intermediate for n_trans transforms
+};
+bool fftn_applicable(const DeconvArgs& a);
+hipError_t fftn_plan_init(FftnPlan& fp, const DeconvArgs& a);  // tables and intermediate (no allocation at run time)
+void fftn_plan_free(FftnPlan& fp);
+// spread grid -> deconvolved modes (overwrites the grid), and modes -> transformed grid
+hipError_t fftn_to_modes(FftnPlan& fp, const DeconvArgs& a, void* grid, void* f, int isign, hipStream_t s);
+hipError_t fftn_to_grid(FftnPlan& fp, const DeconvArgs& a, const void* f, void* grid, int isign, hipStream_t s);
+
 // ---- type 3 (elementwise.hip)
 struct T3State {  // lives in device memory, filled by launch_t3_setup
   double C[3], D[3], gamma[3], h[3];

@@ -412,6 +412,8 @@ struct nufftx_plan_s {
   Fft2Plan fft2;          // fused FFT + deconvolution (2D FP32, power-of-two grids)
   bool fft2_pad = false;      // modes -> grid (type 2 input, adjoint of type 1) fused
   bool fft2_shuffle = false;  // grid -> modes (type 1 output) fused
+  FftnPlan fftn;              // the same on other 2-3-5-smooth grids and in FP64 (type 3: the inner grid)
+  bool fftn_on = false;
   QuadRule quad;
   // type 3
   T3State* t3 = nullptr;
@@ -434,6 +436,7 @@ void plan_free(nufftx_plan p) {
   pointset_free(p->pt);
   fft_free(p->fft);
   fft2_plan_free(p->fft2);
+  fftn_plan_free(p->fftn);
   fft_free(p->fft_in);
   void* bufs[] = {p->grid, p->grid_in, p->fac[0], p->fac[1], p->fac[2], p->fac_in[0], p->fac_in[1], p->fac_in[2],
                   p->t3, p->red, p->xr[0], p->xr[1], p->xr[2], p->sr[0], p->sr[1], p->sr[2], p->pre, p->post,
@@ -550,10 +553,23 @@ DeconvArgs dargs(nufftx_plan p, bool inner) {
     if (e_ != hipSuccess) return fail(NUFFTX_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
+// The mixed-radix passes where they apply (NUFFTX_ROCFFT: rocFFT); inner: the type-3 inner grid.
+int fftn_make(nufftx_plan p, bool inner) {
+  const DeconvArgs a = dargs(p, inner);
+  if (std::getenv("NUFFTX_ROCFFT") || !fftn_applicable(a)) return NUFFTX_OK;
+  if (fftn_plan_init(p->fftn, a) != hipSuccess) return fail(NUFFTX_ERR_ALLOC, "mixed-radix FFT tables and intermediate buffer");
+  p->fftn_on = true;
+  return NUFFTX_OK;
+}
+
 // fine grid -> FFT -> deconvolved modes f (type 1 output stage)
 int grid_to_modes(nufftx_plan p, void* f, int isign) {
   if (p->fft2_shuffle) {
     LAUNCH(fft2_shuffle(p->fft2, dargs(p, false), p->grid, f, isign, p->stream));
+    return NUFFTX_OK;
+  }
+  if (p->fftn_on) {
+    LAUNCH(fftn_to_modes(p->fftn, dargs(p, false), p->grid, f, isign, p->stream));
     return NUFFTX_OK;
   }
   if (int r = fft_exec(p->fft, p->grid, isign, p->stream)) return r;
@@ -565,6 +581,10 @@ int grid_to_modes(nufftx_plan p, void* f, int isign) {
 int modes_to_grid(nufftx_plan p, const void* f, int isign) {
   if (p->fft2_pad) {
     LAUNCH(fft2_pad(p->fft2, dargs(p, false), f, p->grid, isign, p->stream));
+    return NUFFTX_OK;
+  }
+  if (p->fftn_on) {
+    LAUNCH(fftn_to_grid(p->fftn, dargs(p, false), f, p->grid, isign, p->stream));
     return NUFFTX_OK;
   }
   LAUNCH(launch_deconv_pad(dargs(p, false), f, p->grid, p->stream));
@@ -590,8 +610,12 @@ int exec_type3(nufftx_plan p, const void* c, void* f) {
   ga.zero_out = true;
   LAUNCH(launch_spread(ga, p->cbuf, p->grid, p->stream));
   // inner type 2 on the spread grid as CMCL modes (nufft3.py:292, 387, 494-502)
-  LAUNCH(launch_deconv_pad(dargs(p, true), p->grid, p->grid_in, p->stream));
-  if (int r = fft_exec(p->fft_in, p->grid_in, p->isign, p->stream)) return r;
+  if (p->fftn_on) {
+    LAUNCH(fftn_to_grid(p->fftn, dargs(p, true), p->grid, p->grid_in, p->isign, p->stream));
+  } else {
+    LAUNCH(launch_deconv_pad(dargs(p, true), p->grid, p->grid_in, p->stream));
+    if (int r = fft_exec(p->fft_in, p->grid_in, p->isign, p->stream)) return r;
+  }
   LAUNCH(launch_interp(gop(p, p->pt, p->gi), p->grid_in, f, p->stream));
   LAUNCH(launch_cmul_pointwise(p->prec, p->n_trans, p->N, f, p->post, f, p->stream));
   return NUFFTX_OK;
@@ -676,7 +700,6 @@ int nufftx_makeplan(int type, int dim, const int64_t* n_modes, int isign, int64_
       auto ph = phihat(p->g.nf[d], p->quad);
       if ((r = upload_factors(p->fac[d], deconv_factors(ph, p->n_modes[d], modeord), p->prec))) goto fail_out;
     }
-    if ((r = fft_make(p->fft, dim, p->g.nf, n_trans, p->prec))) goto fail_out;
     // Fused FFT + deconvolution passes (Stockham, fft2d.hip) in both directions: on the 2D
     // radial 4M workload (1024^2 grid) nufft2d1 0.198 -> 0.187 ms against rocFFT + the shuffle
     // kernel, nufft2d2 0.160 -> 0.156 ms against the earlier four-step passes.  NUFFTX_ROCFFT
@@ -688,6 +711,8 @@ int nufftx_makeplan(int type, int dim, const int64_t* n_modes, int isign, int64_
       }
       p->fft2_pad = true;
       p->fft2_shuffle = true;
+    } else if ((r = fftn_make(p, false)) || (!p->fftn_on && (r = fft_make(p->fft, dim, p->g.nf, n_trans, p->prec)))) {
+      goto fail_out;
     }
   } else {
     char* gi = nullptr;
@@ -698,7 +723,7 @@ int nufftx_makeplan(int type, int dim, const int64_t* n_modes, int isign, int64_
       auto ph = phihat(p->gi.nf[d], p->quad);
       if ((r = upload_factors(p->fac_in[d], deconv_factors(ph, p->g.nf[d], 0), p->prec))) goto fail_out;
     }
-    if ((r = fft_make(p->fft_in, dim, p->gi.nf, n_trans, p->prec))) goto fail_out;
+    if ((r = fftn_make(p, true)) || (!p->fftn_on && (r = fft_make(p->fft_in, dim, p->gi.nf, n_trans, p->prec)))) goto fail_out;
     if ((r = dev_alloc(p->t3, 1))) goto fail_out;
     if ((r = dev_alloc(p->red, 12 * 256))) goto fail_out;
   }

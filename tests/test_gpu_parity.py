@@ -1009,3 +1009,45 @@ def test_spread64_regions_non_finite(rng):
     touched = R.spread([R.wrap_pi(x)[7:8] for x in coords], np.ones(1, complex), nfs, kp) != 0
     assert np.isposinf(got[1].real[touched]).all()
     assert R.rel_l2(got[1][~touched], ref[1][~touched]) < 1e-13
+
+
+# ------------------------------------------------------------------ mixed-radix FFT + deconvolution passes
+
+
+_FFTN_MODES = [(8,), (9,), (25,), (27,), (75,), (125,), (243,), (270,), (1023,), (2000,),   # one pass per transform
+               (2049,), (5001,), (30375,), (40000,),                                        # axes of two passes
+               (9, 20), (75, 31), (160, 135), (8, 8, 9), (27, 10, 16), (50, 48, 45)]
+
+
+@pytest.mark.parametrize("nm", _FFTN_MODES)
+@pytest.mark.parametrize("prec,modeord,isign,n_trans", [("f32", 0, 1, 1), ("f32", 1, -1, 3), ("f64", 0, -1, 2),
+                                                        ("f64", 1, 1, 1)])
+def test_fftn_vs_rocfft(rng, monkeypatch, nm, prec, modeord, isign, n_trans):
+    """Both directions against plans built with NUFFTX_ROCFFT (rocFFT + the separate deconvolution kernels) on the same
+    points: FFT rounding (2e-6 in FP32 as for the power-of-two passes, 2e-13 in FP64, where the
+    deconvolution amplifies 1e-15 by at most ~100)."""
+    from nufftax_amd._plan import F32, F64, Plan
+
+    dim, M = len(nm), 400
+    rdt, cdt = (torch.float32, torch.complex64) if prec == "f32" else (torch.float64, torch.complex128)
+    eps, tol = (1e-6, 2e-6) if prec == "f32" else (1e-9, 2e-13)
+    xs = [_t(rng.uniform(-np.pi, np.pi, M), rdt) for _ in range(dim)]
+    shape = (n_trans,) + tuple(reversed(nm))
+    c = _t(rng.standard_normal((n_trans, M)) + 1j * rng.standard_normal((n_trans, M)), cdt)
+    f = _t(rng.standard_normal(shape) + 1j * rng.standard_normal(shape), cdt)
+    out = {}
+    for roc in (False, True):
+        if roc:
+            monkeypatch.setenv("NUFFTX_ROCFFT", "1")
+        else:
+            monkeypatch.delenv("NUFFTX_ROCFFT", raising=False)
+        p1, p2 = (Plan.transform(k, dim, nm, n_trans, eps, isign, 2.0, F32 if prec == "f32" else F64, modeord,
+                                 torch.device(DEV, 0)) for k in (1, 2))
+        fo, co = torch.empty(shape, dtype=cdt, device=DEV), torch.empty((n_trans, M), dtype=cdt, device=DEV)
+        p1.setpts(xs)
+        p1.execute(c, fo)
+        p2.setpts(xs)
+        p2.execute(co, f)
+        out[roc] = (_np(fo), _np(co))
+    for got, want in zip(out[False], out[True]):
+        assert R.rel_l2(got, want) < tol
