@@ -9,11 +9,24 @@ namespace nufftx {
 
 namespace {
 
+// 3D FP64: one wave per point straight from the grid instead of LDS tiles, whose FP64 cells leave one block of four
+// waves per CU and whose halo is read again for every bin.  Whole type-2 calls, tiles -> waves: ns = 14 5990 -> 282 us
+// (50k uniform points, 128^3 grid), 6280 -> 1145 (500k), 1119 -> 954 (500k points on 32^3); ns = 10 1407 -> 602 us (500k
+// on 128^3) but 85 -> 94 (50k on 32^3) and 293 -> 461 (500k on 32^3); ns = 8 1205 -> 584 us (500k on 200^3) and 372 ->
+// 394 (on 128^3); ns = 6 200 -> 128 us (50k on 128^3), 648 -> 537 (500k on 200^3) and 219 -> 359 (on 128^3).  So
+// tiles pay from more points per cell the smaller the support is.
+template <typename T, int D>
+bool interp_by_wave(const Geometry& g, int64_t M) {
+  if (D != 3 || !std::is_same<T, double>::value) return false;
+  const int64_t cells = g.grid_cells();
+  return g.ns >= 14 || M <= (g.ns >= 10 ? cells : g.ns == 8 ? cells / 8 : cells / 24);
+}
+
 template <typename T, typename CT, int D>
 hipError_t interp_impl(const GridOpArgs& ga, const void* fw, void* c, hipStream_t s) {
   const SIArgs<T> a = make_si_args<T>(ga);
   size_t lds = 0;
-  const bool tiled = use_tiles(*ga.g, ga.prec, lds);
+  const bool tiled = use_tiles(*ga.g, ga.prec, lds) && !interp_by_wave<T, D>(*ga.g, ga.ps->M);
   const PointSet& ps = *ga.ps;
   GatherOut<T, D, false> o;
   o.val = static_cast<cplx<T>*>(c);

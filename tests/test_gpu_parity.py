@@ -1051,3 +1051,24 @@ def test_fftn_vs_rocfft(rng, monkeypatch, nm, prec, modeord, isign, n_trans):
         out[roc] = (_np(fo), _np(co))
     for got, want in zip(out[False], out[True]):
         assert R.rel_l2(got, want) < tol
+
+
+# ------------------------------------------------------------------ 3D FP64 interpolation, one wave per point
+
+
+@pytest.mark.parametrize("ns", [2, 4, 6, 8, 10, 12, 14, 16])
+@pytest.mark.parametrize("nfs,M", [((16, 18, 20), 1), ((37, 16, 24), 170), ((45, 50, 40), 3001)])
+def test_interp64_vs_oracle(rng, ns, nfs, M):
+    """Either path (tiles or one wave per point, by points per cell) against the oracle, FP64 rounding."""
+    from nufftax_amd._plan import F64, Plan
+
+    kp = R.compute_kernel_params({2: 1e-1, 4: 1e-3, 6: 1e-5, 8: 1e-7, 10: 1e-9, 12: 1e-11, 14: 1e-13, 16: 1e-15}[ns])
+    assert kp.nspread == ns
+    coords = [rng.uniform(-np.pi, np.pi, M) for _ in nfs]
+    fw = rng.standard_normal((2,) + tuple(reversed(nfs))) + 1j * rng.standard_normal((2,) + tuple(reversed(nfs)))
+    plan = Plan.grid_op(3, nfs, ns, kp.beta, kp.c, 2, F64, torch.device(DEV, 0))
+    plan.setpts([_t(x) for x in coords])
+    out = torch.empty((2, M), dtype=torch.complex128, device=DEV)
+    plan.interp(_t(fw), out)
+    for t in range(2):
+        assert R.rel_l2(_np(out)[t], R.interp([R.wrap_pi(x) for x in coords], fw[t], kp)) < 1e-12
