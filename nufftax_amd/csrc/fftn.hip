@@ -504,6 +504,9 @@ hipError_t fftn_run(FftnPlan& fp, const DeconvArgs& a, bool to_grid, const void*
 // Whether every axis is 2-3-5-smooth and fits a pass (1D: or two), and offsets fit 32 bits.
 bool fftn_applicable(const DeconvArgs& a) {
   if (a.dim < 1 || a.dim > 3 || a.from_phihat) return false;
+  // small 3D FP64 grids stay with rocFFT, which transforms two short axes in one launch (type 1 of 2000 points: 64^3 grid
+  // 65 us, 77 with three passes; 80^3 87, 91; 96^3 106, 102)
+  if (a.dim == 3 && a.prec == kF64 && (int64_t)a.nf[0] * a.nf[1] * a.nf[2] < 700000) return false;
   double bytes = a.prec == kF32 ? 8.0 : 16.0;
   for (int d = 0; d < a.dim; ++d) bytes *= a.nf[d];
   if (bytes * (a.dim == 1 ? a.n_trans : 1) > 4294967295.0) return false;
