@@ -39,7 +39,8 @@ struct PointSet {
   int64_t M = 0;
   const void* coord[3] = {nullptr, nullptr, nullptr};
   bool coord_f64 = false;
-  // sort state
+  // sort state (1D point sets are sorted on their first use that needs it, see direct1d.hip)
+  bool sorted = false;
   int NB = 0;        // sort chunks (rows of the histogram matrix)
   int CH = 0;        // points per chunk
   int maxsub = 0;    // max points per subproblem
@@ -233,6 +234,12 @@ constexpr int64_t kSpread64MinPoints = 2048;
 bool spread64_applicable(const Geometry& g, int prec, int64_t M);
 hipError_t spread64_reserve(PointSet& ps, const Geometry& g, int64_t n_trans);  // buffers for M points
 hipError_t launch_spread64(const GridOpArgs& a, const void* c, void* fw, hipStream_t s);
+
+// ---- direct1d.hip: 1D spreading (small grids) and interpolation (any grid) without a sort
+bool spread1d_direct(const Geometry& g);
+bool interp1d_direct(const Geometry& g);
+hipError_t launch_spread1d(const GridOpArgs& a, const void* c, void* fw, hipStream_t s);
+hipError_t launch_interp1d(const GridOpArgs& a, const void* fw, void* c, hipStream_t s);
 
 // ---- elementwise.hip
 hipError_t launch_zero(void* p, int64_t bytes, hipStream_t s);

@@ -36,7 +36,7 @@ hipError_t interp_impl(const GridOpArgs& ga, const void* fw, void* c, hipStream_
   return dispatch_ns(ga.g->ns, [&](auto nsc) -> hipError_t {
     constexpr int NS = decltype(nsc)::value;
     if (tiled) {
-      if constexpr (D >= 2 && std::is_same<T, float>::value && NS <= 8) {
+      if constexpr (std::is_same<T, float>::value && NS <= 8) {
         // 16-byte tile reads (k_gather_wide) unless NUFFTX_INTERP_WIDE=0; rows of an even
         // number of cells keep the reads aligned
         const char* ev = std::getenv("NUFFTX_INTERP_WIDE");
@@ -65,10 +65,10 @@ hipError_t interp_impl(const GridOpArgs& ga, const void* fw, void* c, hipStream_
                          static_cast<const cplx<T>*>(fw), o);
     } else {
       const char* gw = std::getenv("NUFFTX_GLOBAL_WAVE");
-      if (D >= 2 && !(gw && gw[0] == '0')) {
+      if (!(gw && gw[0] == '0')) {
         // one wave per point (four per block)
         const unsigned nblk = (unsigned)((ps.M + 3) / 4);
-        hipLaunchKernelGGL((k_gather_global_wave<T, CT, D == 1 ? 2 : D, NS>), dim3(nblk, (unsigned)ga.n_trans), dim3(256), 0, s, a,
+        hipLaunchKernelGGL((k_gather_global_wave<T, CT, D, NS>), dim3(nblk, (unsigned)ga.n_trans), dim3(256), 0, s, a,
                            static_cast<const cplx<T>*>(fw), static_cast<cplx<T>*>(c));
       } else {
         const unsigned nblk = (unsigned)((ps.M + 255) / 256);
@@ -140,7 +140,6 @@ hipError_t interp_dim(const GridOpArgs& ga, const void* fw, void* c, hipStream_t
     if (interp_win(ga, fw, c, s, err)) return err;
   }
   switch (ga.g->dim) {
-    case 1: return interp_impl<T, CT, 1>(ga, fw, c, s);
     case 2: return interp_impl<T, CT, 2>(ga, fw, c, s);
     case 3: return interp_impl<T, CT, 3>(ga, fw, c, s);
   }
@@ -199,6 +198,7 @@ hipError_t launch_interp_many(const GridOpArgs* gas, int count, const void* cons
 
 hipError_t launch_interp(const GridOpArgs& ga, const void* fw, void* c, hipStream_t s) {
   if (ga.ps->M == 0) return hipSuccess;
+  if (interp1d_direct(*ga.g)) return launch_interp1d(ga, fw, c, s);
   if (ga.prec == kF32) {
     return ga.ps->coord_f64 ? interp_dim<float, double>(ga, fw, c, s) : interp_dim<float, float>(ga, fw, c, s);
   }

@@ -518,8 +518,27 @@ int sort_points(nufftx_plan p, PointSet& ps, const Geometry& g, bool interp, boo
     if (grow_buffer(ps.cmax, ps.cap_cmax, p->n_trans * (1 + std::max<int64_t>(nb, 1)), ps.retired) != hipSuccess)
       return fail(NUFFTX_ERR_ALLOC, "strength bound buffer");
   }
+  ps.sorted = true;
   return NUFFTX_OK;
 }
+
+// Sorts a point set of setpts that has not been sorted yet (1D: direct1d.hip needs no sort).
+int need_sorted(nufftx_plan p, bool inner) {
+  PointSet& ps = inner ? p->pt : p->ps;
+  return ps.sorted ? NUFFTX_OK : sort_points(p, ps, inner ? p->gi : p->g, inner || p->type != 1, !inner && p->type != 2);
+}
+
+// setpts: sort now, unless neither the forward use nor (1D) anything else needs it yet
+int set_points(nufftx_plan p, bool inner) {
+  const Geometry& g = inner ? p->gi : p->g;
+  (inner ? p->pt : p->ps).sorted = false;
+  const bool spreads = !inner && (p->type == 1 || p->type == 3);
+  if (g.dim == 1 && interp1d_direct(g) && (!spreads || spread1d_direct(g))) return NUFFTX_OK;
+  return need_sorted(p, inner);
+}
+
+// before a spread from the plan's points, and before a gather of coordinate gradients
+int spread_ready(nufftx_plan p) { return spread1d_direct(p->g) ? NUFFTX_OK : need_sorted(p, false); }
 
 GridOpArgs gop(nufftx_plan p, const PointSet& ps, const Geometry& g) {
   GridOpArgs a;
@@ -592,6 +611,7 @@ int modes_to_grid(nufftx_plan p, const void* f, int isign) {
 }
 
 int exec_type1(nufftx_plan p, const void* c, void* f, int isign) {
+  if (int r = spread_ready(p)) return r;
   GridOpArgs ga = gop(p, p->ps, p->g);
   ga.zero_out = true;
   LAUNCH(launch_spread(ga, c, p->grid, p->stream));
@@ -783,7 +803,7 @@ int nufftx_setpts(nufftx_plan p, int64_t M, const void* x, const void* y, const 
     p->ps.M = M;
     for (int d = 0; d < 3; ++d) p->ps.coord[d] = d < p->dim ? xs[d] : nullptr;
     p->ps.coord_f64 = p->prec == kF64;
-    if (int r = sort_points(p, p->ps, p->g, p->type != 1, p->type != 2)) return r;
+    if (int r = set_points(p, false)) return r;
     p->pts_set = true;
     return NUFFTX_OK;
   }
@@ -818,8 +838,8 @@ int nufftx_setpts(nufftx_plan p, int64_t M, const void* x, const void* y, const 
     p->pt.coord[d] = d < p->dim ? p->sr[d] : nullptr;
   }
   p->ps.coord_f64 = p->pt.coord_f64 = true;
-  if ((r = sort_points(p, p->ps, p->g, false, true))) return r;
-  if ((r = sort_points(p, p->pt, p->gi, true, false))) return r;
+  if ((r = set_points(p, false))) return r;
+  if ((r = set_points(p, true))) return r;
   p->pts_set = true;
   return NUFFTX_OK;
 }
@@ -907,6 +927,7 @@ int nufftx_vjp(nufftx_plan p, const void* src, const void* g, void* grad_src, vo
     // G = FFT_{-isign}(pad(g / phihat)) -- adjoint of deconvolve-shuffle and FFT
     if (int r = modes_to_grid(p, g, s)) return r;
     if (want_coord) {
+      if (int r = need_sorted(p, false)) return r;
       LAUNCH(launch_interp_grad(gop(p, p->ps, p->g), p->grid, src, grad_src, gc, p->stream));
     } else if (grad_src) {
       LAUNCH(launch_interp(gop(p, p->ps, p->g), p->grid, grad_src, p->stream));
@@ -916,6 +937,7 @@ int nufftx_vjp(nufftx_plan p, const void* src, const void* g, void* grad_src, vo
   // type 2
   if (want_coord) {
     if (int r = modes_to_grid(p, src, p->isign)) return r;
+    if (int r = need_sorted(p, false)) return r;
     LAUNCH(launch_interp_grad(gop(p, p->ps, p->g), p->grid, g, nullptr, gc, p->stream));
   }
   if (grad_src) return exec_type1(p, g, grad_src, s);
@@ -934,6 +956,7 @@ int nufftx_spread(nufftx_plan p, const void* c, void* fw) {
   if (int r = check_plan(p)) return r;
   if (!p->pts_set) return fail(NUFFTX_ERR_STATE, "setpts has not been called");
   if (!fw || (!c && p->M > 0)) return fail(NUFFTX_ERR_INVALID_ARG, "null data pointer");
+  if (int r = spread_ready(p)) return r;
   GridOpArgs ga = gop(p, p->ps, p->g);
   ga.zero_out = true;
   LAUNCH(launch_spread(ga, c, fw, p->stream));
@@ -944,6 +967,7 @@ int nufftx_spread_add(nufftx_plan p, const void* c, void* fw) {
   if (int r = check_plan(p)) return r;
   if (!p->pts_set) return fail(NUFFTX_ERR_STATE, "setpts has not been called");
   if (!fw || (!c && p->M > 0)) return fail(NUFFTX_ERR_INVALID_ARG, "null data pointer");
+  if (int r = spread_ready(p)) return r;
   LAUNCH(launch_spread(gop(p, p->ps, p->g), c, fw, p->stream));
   return NUFFTX_OK;
 }
@@ -963,6 +987,7 @@ int nufftx_gather_grad(nufftx_plan p, const void* G, const void* P, void* gval, 
   const bool want_coord = gc[0] || gc[1] || gc[2];
   if (!G || (want_coord && !P)) return fail(NUFFTX_ERR_INVALID_ARG, "null data pointer");
   if (want_coord) {
+    if (int r = need_sorted(p, false)) return r;
     LAUNCH(launch_interp_grad(gop(p, p->ps, p->g), G, P, gval, gc, p->stream));
   } else if (gval) {
     LAUNCH(launch_interp(gop(p, p->ps, p->g), G, gval, p->stream));
@@ -984,6 +1009,8 @@ int nufftx_get_sort_info(nufftx_plan p, int inner, int* nbins, int* bin_size, in
 int nufftx_copy_sort(nufftx_plan p, int inner, int32_t* perm, int32_t* bin_start) {
   if (int r = check_plan(p)) return r;
   if (!p->pts_set) return fail(NUFFTX_ERR_STATE, "setpts has not been called");
+  if (!inner || p->type == 3)
+    if (int r = need_sorted(p, inner != 0)) return r;
   const PointSet& ps = inner ? p->pt : p->ps;
   const Geometry& g = inner ? p->gi : p->g;
   if (perm && ps.M > 0) HIPCHK(hipMemcpyAsync(perm, ps.perm, ps.M * sizeof(int32_t), hipMemcpyDeviceToDevice, p->stream));

@@ -310,6 +310,7 @@ hipError_t launch_spread_many(const GridOpArgs* gas, int count, const void* cons
 hipError_t launch_spread(const GridOpArgs& ga, const void* c, void* fw, hipStream_t s) {
   if (ga.ps->M == 0)
     return ga.zero_out ? launch_zero(fw, ga.n_trans * ga.g->grid_cells() * (ga.prec == kF32 ? 8 : 16), s) : hipSuccess;
+  if (spread1d_direct(*ga.g)) return launch_spread1d(ga, c, fw, s);
   if (ga.prec == kF32) {
     return ga.ps->coord_f64 ? spread_dim<float, double>(ga, c, fw, s) : spread_dim<float, float>(ga, c, fw, s);
   }

@@ -1072,3 +1072,55 @@ def test_interp64_vs_oracle(rng, ns, nfs, M):
     plan.interp(_t(fw), out)
     for t in range(2):
         assert R.rel_l2(_np(out)[t], R.interp([R.wrap_pi(x) for x in coords], fw[t], kp)) < 1e-12
+
+
+# ------------------------------------------------------------------ 1D without a sort
+
+
+@pytest.mark.parametrize("prec,ns", [("f32", 2), ("f32", 8), ("f64", 6), ("f64", 16)])
+@pytest.mark.parametrize("nf,M", [(4, 3), (16, 1), (100, 2048), (2048, 2049), (4096, 5000), (4097, 5000), (60000, 3001)])
+def test_direct1d_vs_oracle(rng, prec, ns, nf, M):
+    """Spread (overwriting and adding) and interp around the sizes where the path changes: one block and several, LDS
+    and memory, sorted spreading above 4096 cells.  Tolerances of the other spread / interp tests."""
+    from nufftax_amd._plan import F32, F64, Plan
+
+    rdt, cdt, tol = (np.float32, np.complex64, 2e-6) if prec == "f32" else (np.float64, np.complex128, 1e-12)
+    kp = R.compute_kernel_params({2: 1e-1, 6: 1e-5, 8: 1e-7, 16: 1e-15}[ns])
+    assert kp.nspread == ns
+    x = rng.uniform(-np.pi, np.pi, M).astype(rdt)
+    c = (rng.standard_normal((2, M)) + 1j * rng.standard_normal((2, M))).astype(cdt)
+    g = (rng.standard_normal((2, nf)) + 1j * rng.standard_normal((2, nf))).astype(cdt)
+    plan = Plan.grid_op(1, (nf,), ns, kp.beta, kp.c, 2, F32 if prec == "f32" else F64, torch.device(DEV, 0))
+    plan.setpts([_t(x)])
+    xw = [x.astype(np.float64)]
+    fw = _t(np.full((2, nf), np.nan, cdt))
+    plan.spread(_t(c), fw)
+    out = torch.empty((2, M), dtype=torch.complex64 if prec == "f32" else torch.complex128, device=DEV)
+    plan.interp(_t(g), out)
+    if prec == "f64" and nf > 4097:
+        # the oracle rounds its folded positions (7e-12 cells at 60000 cells), the library's FMA does not: the
+        # direct interpolation is held to be the transpose of the sorted spread instead
+        for t in range(2):
+            a, b = np.sum(_np(out)[t] * c[t]), np.sum(g[t] * _np(fw)[t])
+            assert abs(a - b) < tol * np.linalg.norm(_np(out)[t]) * np.linalg.norm(c[t])
+        return
+    want = np.stack([R.spread(xw, c[t].astype(complex), (nf,), kp) for t in range(2)])
+    assert R.rel_l2(_np(fw), want) < tol
+    assert R.rel_l2(_np(out), np.stack([R.interp(xw, g[t].astype(complex), kp) for t in range(2)])) < tol
+    fw = _t(g)
+    plan.spread_add(_t(c), fw)
+    assert R.rel_l2(_np(fw), want + g) < tol
+
+
+def test_direct1d_sorts_when_asked(rng):
+    """A 1D plan that has not needed its sort makes it for the sort state and for coordinate gradients."""
+    from nufftax_amd._plan import F32, Plan
+
+    x = rng.uniform(-np.pi, np.pi, 5000).astype(np.float32)
+    plan = Plan.transform(1, 1, (1000,), 1, 1e-6, 1, 2.0, F32, 0, torch.device(DEV, 0))
+    plan.setpts([_t(x)])
+    perm, bst, nbins, bs, _ = plan.sort_state()
+    keys = R.bin_keys([x.astype(np.float64)], [plan.grid_size(0)], bs[:1])
+    ref_perm, ref_off = R.bin_sort(keys, nbins)
+    np.testing.assert_array_equal(_np(perm).astype(np.int64), ref_perm)
+    np.testing.assert_array_equal(_np(bst).astype(np.int64), ref_off)
