@@ -102,6 +102,11 @@ int nufftx_execute(nufftx_plan plan, void* c, void* f);
 /* Same as execute with the exponent sign overridden (type 1/2 only). */
 int nufftx_execute_sign(nufftx_plan plan, void* c, void* f, int isign);
 
+/* nufftx_set_stream + nufftx_setpts + nufftx_execute_sign in one call (new points on every call): same arguments, checks
+ * and results.  Not for plans of nufftx_plan_acquire, which keep their stream. */
+int nufftx_run(nufftx_plan plan, void* stream, int64_t M, const void* x, const void* y, const void* z, int64_t N, const void* s,
+               const void* t, const void* u, void* c, void* f, int isign);
+
 /*
  * Execute count plans (all type 1 or all type 2, each with its own points, grid size and
  * isign): plan i runs c[i] -> f[i] (type 1) or f[i] -> c[i] (type 2), as nufftx_execute.

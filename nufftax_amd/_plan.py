@@ -26,8 +26,14 @@ from . import _lib
 from ._lib import F32, F64, check, lib, ptr
 
 
+# the current stream's handle without a Stream object (2 us of a small call, three times)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    if _raw_stream is None or device.index is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 def _tensor_key(t):
@@ -107,6 +113,20 @@ class Plan:
             "nufftx_setpts",
         )
         self._pts_key = key
+        self._pts_refs = (coords, targets)
+        self.M, self.N = M, N
+
+    def run(self, coords, targets, c, f, isign):
+        """setpts + execute in one library call: the points are sorted on every call (as setpts without reuse)."""
+        M = coords[0].numel()
+        N = targets[0].numel() if targets else 0
+        xs = [t.data_ptr() for t in coords] + [None] * (3 - len(coords))
+        ss = [t.data_ptr() for t in targets] + [None] * (3 - len(targets))
+        self._pts_key = None
+        check(
+            lib().nufftx_run(self.h, _stream_handle(self.device), M, *xs, N, *ss, c.data_ptr(), f.data_ptr(), isign),
+            "nufftx_run",
+        )
         self._pts_refs = (coords, targets)
         self.M, self.N = M, N
 
@@ -223,8 +243,8 @@ CACHE = PlanCache()
 def transform_plan(kind, dim, n_modes, n_trans, eps, isign, upsampfac, prec, device, modeord=0) -> Plan:
     device = torch.device(device)
     stream = _stream_handle(device)
-    key = ("t", kind, dim, tuple(int(v) for v in n_modes), int(n_trans), float(eps), int(isign), float(upsampfac),
-           prec, modeord, device.index, stream)
+    key = ("t", kind, dim, tuple(n_modes), n_trans, float(eps), int(isign), float(upsampfac), prec, modeord,
+           device.index, stream)
     return CACHE.get(key, lambda: Plan.transform(kind, dim, n_modes, n_trans, eps, isign, upsampfac, prec, modeord,
                                                  device))
 

@@ -861,6 +861,13 @@ int nufftx_execute(nufftx_plan p, void* c, void* f) {
   return nufftx_execute_sign(p, c, f, p->isign);
 }
 
+int nufftx_run(nufftx_plan p, void* stream, int64_t M, const void* x, const void* y, const void* z, int64_t N, const void* s,
+               const void* t, const void* u, void* c, void* f, int isign) {
+  if (int r = nufftx_set_stream(p, stream)) return r;
+  if (int r = nufftx_setpts(p, M, x, y, z, N, s, t, u)) return r;
+  return nufftx_execute_sign(p, c, f, isign);
+}
+
 int nufftx_execute_many(int count, const nufftx_plan* plans, void* const* c, void* const* f) {
   if (count < 1 || !plans || !c || !f) return fail(NUFFTX_ERR_INVALID_ARG, "execute_many: empty or null batch");
   for (int i = 0; i < count; ++i) {

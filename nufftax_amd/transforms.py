@@ -109,7 +109,8 @@ def _complex_dtype_of(t: torch.Tensor) -> torch.dtype:
 def _coords(coords, rdt, device, M):
     out = []
     for x in coords:
-        x = x.to(device=device, dtype=rdt)
+        if x.dtype is not rdt or x.device != device:
+            x = x.to(device=device, dtype=rdt)
         if x.ndim != 1 or x.shape[0] != M:
             raise ValueError(f"coordinate arrays must have shape ({M},), got {tuple(x.shape)}")
         out.append(x.contiguous())
@@ -144,8 +145,7 @@ def _raw_type1(meta: _Meta, c: torch.Tensor, coords, isign=None, upsampfac=None)
     for s, e in _chunks(n_trans):
         plan = transform_plan(1, dim, meta.n_modes, e - s, meta.eps, isign, uf, prec, dev)
         with plan.lock:
-            plan.setpts(xs)
-            plan.execute(cc[s:e], out[s:e], isign)
+            plan.run(xs, (), *((cc, out) if e - s == n_trans else (cc[s:e], out[s:e])), isign)
     return out.reshape(lead + tuple(reversed(meta.n_modes))).to(c.dtype)
 
 
@@ -165,8 +165,7 @@ def _raw_type2(meta: _Meta, f: torch.Tensor, coords, isign=None, upsampfac=None)
     for s, e in _chunks(n_trans):
         plan = transform_plan(2, dim, nm, e - s, meta.eps, isign, uf, prec, dev)
         with plan.lock:
-            plan.setpts(xs)
-            plan.execute(out[s:e], ff[s:e], isign)
+            plan.run(xs, (), *((out, ff) if e - s == n_trans else (out[s:e], ff[s:e])), isign)
     return out.reshape(lead + (M,)).to(f.dtype)
 
 
@@ -186,8 +185,7 @@ def _raw_type3(meta: _Meta, c: torch.Tensor, coords, targets, isign=None):
     for s, e in _chunks(n_trans):
         plan = transform_plan(3, dim, meta.n_modes, e - s, meta.eps, isign, meta.upsampfac, prec, dev)
         with plan.lock:
-            plan.setpts(xs, ss)
-            plan.execute(cc[s:e], out[s:e])
+            plan.run(xs, ss, cc[s:e], out[s:e], isign)
     return out.reshape(lead + (N,)).to(c.dtype)
 
 
@@ -499,8 +497,14 @@ def _run(fn, meta, src, *ts):
 # ---------------------------------------------------------------- input normalisation
 
 
+def _as_is(out):
+    return out
+
+
 def _prepare(arrays):
     """Convert to tensors on the GPU; returns (tensors, restore_fn)."""
+    if all(type(a) is torch.Tensor and a.is_cuda for a in arrays) and all(a.device == arrays[0].device for a in arrays):
+        return arrays, _as_is
     was_numpy = any(isinstance(a, np.ndarray) for a in arrays)
     ts = [_to_tensor(a) for a in arrays]
     dev = _target_device(ts)
