@@ -76,6 +76,15 @@ __device__ __forceinline__ int wrap_idx(int g, int n) {
   return g < 0 ? g + n : g;
 }
 
+// wrap_idx for indices near the grid (tiles reach less than a grid past its ends, but for grids smaller than a tile):
+// two selects, a remainder only where they are not enough
+__device__ __forceinline__ int wrap_near(int g, int n) {
+  g += g < 0 ? n : 0;
+  g -= g >= n ? n : 0;
+  if ((unsigned)g >= (unsigned)n) g = wrap_idx(g, n);
+  return g;
+}
+
 template <int D>
 __device__ __forceinline__ void tile_origin(const int4& sd, const int (&bs)[3], const int (&nb)[3], int half,
                                             int (&org)[3]) {

@@ -1074,6 +1074,42 @@ def test_interp64_vs_oracle(rng, ns, nfs, M):
         assert R.rel_l2(_np(out)[t], R.interp([R.wrap_pi(x) for x in coords], fw[t], kp)) < 1e-12
 
 
+# ------------------------------------------------------------------ 3D FP32 interpolation on the matrix cores
+
+
+@pytest.mark.parametrize(
+    "nfs,M,spread",
+    [((16, 16, 16), 1, 1.0), ((16, 18, 20), 17, 1.0), ((45, 37, 50), 900, 1.0), ((64, 32, 48), 3001, 1.0), ((40, 40, 40), 2500, 0.02)],
+)
+def test_gather3_vs_oracle(rng, nfs, M, spread):
+    """ns = 8 windows against the oracle: one point and whole subproblems (2500 points in a few cells), grids as small
+    as a bin and of odd sizes (tiles wrap), two transforms; then with one cell NaN, which only its points may see.
+    Tolerance of the other FP32 spread / interp tests."""
+    from nufftax_amd._plan import F32, Plan
+
+    kp = R.compute_kernel_params(1e-7)
+    assert kp.nspread == 8
+    coords = [(spread * rng.uniform(-np.pi, np.pi, M)).astype(np.float32) for _ in nfs]
+    shape = (2,) + tuple(reversed(nfs))
+    fw = (rng.standard_normal(shape) + 1j * rng.standard_normal(shape)).astype(np.complex64)
+    plan = Plan.grid_op(3, nfs, 8, kp.beta, kp.c, 2, F32, torch.device(DEV, 0))
+    plan.setpts([_t(x) for x in coords])
+    out = torch.empty((2, M), dtype=torch.complex64, device=DEV)
+    xs = [R.wrap_pi(x.astype(np.float64)) for x in coords]
+    plan.interp(_t(fw), out)
+    want = [R.interp(xs, fw[t].astype(np.complex128), kp) for t in range(2)]
+    for t in range(2):
+        assert R.rel_l2(_np(out)[t], want[t]) < 2e-6
+    fw[0, nfs[2] // 2, nfs[1] // 2, nfs[0] // 2] = np.nan
+    plan.interp(_t(fw), out)
+    one = R.interp(xs, fw[0].astype(np.complex128), kp)
+    assert np.array_equal(np.isnan(_np(out)[0]), np.isnan(one))
+    seen = np.isnan(one)
+    if not seen.all():
+        assert R.rel_l2(_np(out)[0][~seen], one[~seen]) < 2e-6
+    assert R.rel_l2(_np(out)[1], want[1]) < 2e-6
+
+
 # ------------------------------------------------------------------ 1D without a sort
 
 
