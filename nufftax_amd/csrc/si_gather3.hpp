@@ -12,7 +12,7 @@
 // 64 rows a load: 1937 us where the thread-per-point gather takes 1170; 8M points.)
 //
 // What bounds the thread-per-point gather (k_gather_wide) is its LDS: 8 ns^3 bytes and a quarter per point, at scattered
-// rows (8M clustered points, ns = 8, 256^3 modes: 41 GB, 520 us at the LDS's rate, 1170 measured).  Here a point's cells
+// rows (8M clustered points, ns = 8, 128^3 modes: 41 GB, 520 us at the LDS's rate, 1170 measured).  Here a point's cells
 // are shared by its group, and the vector instructions bound it: about 400 a group beside its 48 MFMAs (510 us at full
 // issue); 950 us measured with two blocks per CU (78 KB of LDS, 187 registers).
 //

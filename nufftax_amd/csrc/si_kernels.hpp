@@ -97,19 +97,59 @@ __device__ __forceinline__ void tile_origin(const int4& sd, const int (&bs)[3], 
   }
 }
 
+// Walk of one thread over a tile's cells first, first + step, ..: the cell's coordinates follow by additions and two
+// compares.  (Taking each cell apart by itself, two 64-bit and three 32-bit divisions a cell: the 3D window spread of 8M
+// clustered points 1419 us, now 1345; the 2D gather of 4M radial points 69.0, now 65.5.)
 template <int D>
-__device__ __forceinline__ int64_t tile_cell_to_global(int64_t cell, const int (&tile)[3], const int (&org)[3],
-                                                       const int (&nf)[3]) {
-  const int l0 = (int)(cell % tile[0]);
-  int64_t r = cell / tile[0];
-  const int l1 = (int)(r % tile[1]);
-  const int l2 = (int)(r / tile[1]);
-  const int g0 = wrap_idx(org[0] + l0, nf[0]);
-  if (D == 1) return g0;
-  const int g1 = wrap_idx(org[1] + l1, nf[1]);
-  if (D == 2) return (int64_t)g1 * nf[0] + g0;
-  const int g2 = wrap_idx(org[2] + l2, nf[2]);
-  return ((int64_t)g2 * nf[1] + g1) * nf[0] + g0;
+struct TileWalk {
+  int l0, l1, l2, s0, s1, s2, t0, t1;
+  __device__ __forceinline__ TileWalk(int first, int step, int tile0, int tile1) : t0(tile0), t1(tile1) {
+    split(first, l0, l1, l2);
+    split(step, s0, s1, s2);
+  }
+  __device__ __forceinline__ void split(int c, int& x, int& y, int& z) const {
+    const int r = c / t0;
+    x = c - r * t0;
+    z = D == 3 ? r / t1 : 0;
+    y = D == 3 ? r - z * t1 : r;
+  }
+  __device__ __forceinline__ void next() {
+    l0 += s0;
+    const int c0 = l0 >= t0;
+    l0 -= c0 ? t0 : 0;
+    l1 += s1 + c0;
+    if (D == 3) {
+      const int c1 = l1 >= t1;
+      l1 -= c1 ? t1 : 0;
+      l2 += s2 + c1;
+    }
+  }
+  // grid index of the cell
+  __device__ __forceinline__ int64_t at(const int (&org)[3], const int (&nf)[3]) const {
+    const int g0 = wrap_near(org[0] + l0, nf[0]);
+    if (D == 1) return g0;
+    const int g1 = wrap_near(org[1] + l1, nf[1]);
+    if (D == 2) return (int64_t)g1 * nf[0] + g0;
+    const int g2 = wrap_near(org[2] + l2, nf[2]);
+    return ((int64_t)g2 * nf[1] + g1) * nf[0] + g0;
+  }
+};
+
+// the tile's cells from the grid, four loads in flight per thread
+template <int D, typename T>
+__device__ __forceinline__ void load_tile(const SIArgs<T>& a, const cplx<T>* __restrict__ fT, const int (&org)[3],
+                                          cplx<T>* tile) {
+  const int n = (int)a.tile_cells, step = (int)blockDim.x;
+  TileWalk<D> w(threadIdx.x, step, a.tile[0], a.tile[1]);
+  for (int cell = threadIdx.x; cell < n; cell += 4 * step) {
+    cplx<T> v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u, w.next())
+      if (cell + u * step < n) v[u] = fT[w.at(org, a.nf)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (cell + u * step < n) tile[cell + u * step] = v[u];
+  }
 }
 
 // Rotated support walk for spreading.  Lane l visits support offset
@@ -293,7 +333,8 @@ __global__ void __launch_bounds__(256) k_spread_tiled(SIArgs<T> a, const cplx<T>
   }
   __syncthreads();
   cplx<T>* fT = fw + (int64_t)tr * a.grid_cells;
-  for (int64_t cell = threadIdx.x; cell < a.tile_cells; cell += blockDim.x) {
+  TileWalk<D> walk(threadIdx.x, blockDim.x, a.tile[0], a.tile[1]);
+  for (int cell = threadIdx.x; cell < (int)a.tile_cells; cell += blockDim.x, walk.next()) {
     T vr, vi;
     if constexpr (kFixed) {
       const long long ir = (long long)sre[cell], ii = (long long)sim[cell];
@@ -305,7 +346,7 @@ __global__ void __launch_bounds__(256) k_spread_tiled(SIArgs<T> a, const cplx<T>
       vi = sim[cell];
       if (vr == (T)0 && vi == (T)0) continue;
     }
-    const int64_t gi = tile_cell_to_global<D>(cell, a.tile, org, a.nf);
+    const int64_t gi = walk.at(org, a.nf);
     atomic_add_global(&fT[gi].re, vr);
     atomic_add_global(&fT[gi].im, vi);
   }
@@ -516,7 +557,8 @@ __device__ __forceinline__ void spread_banked_block(const SIArgs<float>& a, int 
   }
   __syncthreads();
   cplx<float>* fT = fw + (int64_t)tr * a.grid_cells;
-  for (int64_t cell = threadIdx.x; cell < a.tile_cells; cell += blockDim.x) {
+  TileWalk<D> walk(threadIdx.x, blockDim.x, a.tile[0], a.tile[1]);
+  for (int cell = threadIdx.x; cell < (int)a.tile_cells; cell += blockDim.x, walk.next()) {
     long long ir, ii;
     if constexpr (PK) {
       unpack_re_im(sre[cell], ir, ii);
@@ -527,7 +569,7 @@ __device__ __forceinline__ void spread_banked_block(const SIArgs<float>& a, int 
     if (finite && ir == 0 && ii == 0) continue;
     const float vr = finite ? (float)((double)ir * inv_scale) : NAN;
     const float vi = finite ? (float)((double)ii * inv_scale) : NAN;
-    const int64_t gi = tile_cell_to_global<D>(cell, a.tile, org, a.nf);
+    const int64_t gi = walk.at(org, a.nf);
     atomic_add_global(&fT[gi].re, vr);
     atomic_add_global(&fT[gi].im, vi);
   }
@@ -796,8 +838,7 @@ __device__ __forceinline__ void gather_tiled_block(const SIArgs<T>& a, const cpl
   int org[3];
   tile_origin<D>(sd4, a.bs, a.nb, NS / 2, org);
   const cplx<T>* fT = fw + (int64_t)tr * a.grid_cells;
-  for (int64_t cell = threadIdx.x; cell < a.tile_cells; cell += blockDim.x)
-    tile[cell] = fT[tile_cell_to_global<D>(cell, a.tile, org, a.nf)];
+  load_tile<D>(a, fT, org, tile);
   __syncthreads();
   const int t0 = a.tile[0], t1 = a.tile[1];
   for (int j = threadIdx.x; j < sd4.z; j += blockDim.x) {
@@ -860,8 +901,7 @@ __global__ void __launch_bounds__(256) k_gather_wide(SIArgs<float> a, const cplx
   int org[3];
   tile_origin<D>(sd4, a.bs, a.nb, NS / 2, org);
   const cplx<float>* fT = fw + (int64_t)tr * a.grid_cells;
-  for (int64_t cell = threadIdx.x; cell < a.tile_cells; cell += blockDim.x)
-    tile[cell] = fT[tile_cell_to_global<D>(cell, a.tile, org, a.nf)];
+  load_tile<D>(a, fT, org, tile);
   if (threadIdx.x < 2) tile[a.tile_cells + threadIdx.x] = cplx<float>{0.0f, 0.0f};
   __syncthreads();
   const int t0 = a.tile[0], t1 = a.tile[1];
@@ -960,8 +1000,7 @@ __global__ void __launch_bounds__(256) k_gather_wide_deriv(SIArgs<float> a, cons
   int org[3];
   tile_origin<D>(sd4, a.bs, a.nb, NS / 2, org);
   const cplx<float>* fT = fw + (int64_t)tr * a.grid_cells;
-  for (int64_t cell = threadIdx.x; cell < a.tile_cells; cell += blockDim.x)
-    tile[cell] = fT[tile_cell_to_global<D>(cell, a.tile, org, a.nf)];
+  load_tile<D>(a, fT, org, tile);
   if (threadIdx.x < 2) tile[a.tile_cells + threadIdx.x] = cplx<float>{0.0f, 0.0f};
   __syncthreads();
   const int t0 = a.tile[0], t1 = a.tile[1];

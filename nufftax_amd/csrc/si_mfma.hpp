@@ -230,14 +230,14 @@ __global__ void __launch_bounds__(kMfmaThreads) k_spread_mfma2d(SIArgs<float> a,
   __syncthreads();
   // ---- flush non-zero cells to the fine grid
   cplx<float>* fT = fw + (int64_t)tr * a.grid_cells;
-  const int tile3[3] = {T, T, 1};
-  for (int cell = tid; cell < T * T; cell += kMfmaThreads) {
-    const int l = (cell / T) * TP + cell % T;
+  TileWalk<2> walk(tid, kMfmaThreads, T, T);
+  for (int cell = tid; cell < T * T; cell += kMfmaThreads, walk.next()) {
+    const int l = walk.l1 * TP + walk.l0;
     const long long ir = (long long)sre[l], ii = (long long)sim[l];
     if (finite && ir == 0 && ii == 0) continue;
     const float vr = finite ? (float)((double)ir * inv_scale) : NAN;
     const float vi = finite ? (float)((double)ii * inv_scale) : NAN;
-    const int64_t gi = tile_cell_to_global<2>(cell, tile3, org, a.nf);
+    const int64_t gi = walk.at(org, a.nf);
     atomic_add_global(&fT[gi].re, vr);
     atomic_add_global(&fT[gi].im, vi);
   }
@@ -312,11 +312,11 @@ __global__ void __launch_bounds__(kMfmaThreads) k_interp_mfma2d(SIArgs<float> a,
   int org[3];
   tile_origin<2>(sd, a.bs, a.nb, NS / 2, org);
   const cplx<float>* fT = fw + (int64_t)tr * a.grid_cells;
-  const int tile3[3] = {T, T, 1};
-  for (int cell = tid; cell < T * T; cell += kMfmaThreads) {
-    const int64_t gi = tile_cell_to_global<2>(cell, tile3, org, a.nf);
+  TileWalk<2> walk(tid, kMfmaThreads, T, T);
+  for (int cell = tid; cell < T * T; cell += kMfmaThreads, walk.next()) {
+    const int64_t gi = walk.at(org, a.nf);
     const cplx<float> v = fT[gi];
-    const int l = (cell / T) * TP + cell % T;
+    const int l = walk.l1 * TP + walk.l0;
     tre[l] = v.re;
     tim[l] = v.im;
   }

@@ -323,8 +323,8 @@ __global__ void __launch_bounds__(kWinThreads) k_spread_win2d(SIArgs<float> a, i
 
   // ---- 3. flush the tile's non-zero cells to the fine grid
   cplx<float>* fT = fw + (int64_t)tr * a.grid_cells;
-  const int tile3[3] = {T, T, 1};
-  for (int cell = tid; cell < TC; cell += kWinThreads) {
+  TileWalk<2> walk(tid, kWinThreads, T, T);
+  for (int cell = tid; cell < TC; cell += kWinThreads, walk.next()) {
     long long ir, ii;
     if constexpr (PK) {
       unpack_re_im(sre[cell], ir, ii);
@@ -335,7 +335,7 @@ __global__ void __launch_bounds__(kWinThreads) k_spread_win2d(SIArgs<float> a, i
     if (finite && ir == 0 && ii == 0) continue;
     const float vr = finite ? (float)((double)ir * inv_scale) : NAN;
     const float vi = finite ? (float)((double)ii * inv_scale) : NAN;
-    const int64_t gi = tile_cell_to_global<2>(cell, tile3, org, a.nf);
+    const int64_t gi = walk.at(org, a.nf);
     atomic_add_global(&fT[gi].re, vr);
     atomic_add_global(&fT[gi].im, vi);
   }
@@ -630,13 +630,13 @@ __global__ void __launch_bounds__(kWhThreads) k_spread_win2dh(SIArgs<float> a, i
 
   // ---- 3. flush the tile's non-zero cells to the fine grid
   cplx<float>* fT = fw + (int64_t)tr * a.grid_cells;
-  const int tile3[3] = {T, T, 1};
-  for (int cell = tid; cell < TC; cell += kWhThreads) {
+  TileWalk<2> walk(tid, kWhThreads, T, T);
+  for (int cell = tid; cell < TC; cell += kWhThreads, walk.next()) {
     const long long ir = (long long)sre[cell], ii = (long long)sim[cell];
     if (finite && ir == 0 && ii == 0) continue;
     const float vr = finite ? (float)((double)ir * inv_scale) : NAN;
     const float vi = finite ? (float)((double)ii * inv_scale) : NAN;
-    const int64_t gi = tile_cell_to_global<2>(cell, tile3, org, a.nf);
+    const int64_t gi = walk.at(org, a.nf);
     atomic_add_global(&fT[gi].re, vr);
     atomic_add_global(&fT[gi].im, vi);
   }
@@ -711,7 +711,6 @@ __global__ void __launch_bounds__(kWiThreads) k_interp_win2dh(SIArgs<float> a, i
   int4* meta = reinterpret_cast<int4*>(rowy + kWiRowF);  // {y read index, x read index, output index, -}
   int org[3];
   tile_origin<2>(sd, a.bs, a.nb, NS / 2, org);
-  const int tile3[3] = {T, T, 1};
   const cplx<float>* fT = fw + (int64_t)tr * a.grid_cells;
   if (tid == 0) smax = 0u;
   for (int e = tid; e < kWiPpt * W * 16; e += kWiThreads) wcnt[e] = 0;
@@ -723,8 +722,9 @@ __global__ void __launch_bounds__(kWiThreads) k_interp_win2dh(SIArgs<float> a, i
   __syncthreads();
   // ---- 1. tile and its max |re|, |im|
   unsigned mymax = 0;
-  for (int cell = tid; cell < TC; cell += kWiThreads) {
-    const cplx<float> v = fT[tile_cell_to_global<2>(cell, tile3, org, a.nf)];
+  TileWalk<2> walk(tid, kWiThreads, T, T);
+  for (int cell = tid; cell < TC; cell += kWiThreads, walk.next()) {
+    const cplx<float> v = fT[walk.at(org, a.nf)];
     tile[cell] = v;
     mymax = max(mymax, max(__float_as_uint(fabsf(v.re)), __float_as_uint(fabsf(v.im))));
   }

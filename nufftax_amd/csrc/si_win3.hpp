@@ -331,9 +331,11 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
   if (g1 > g0 && finite) flush(s);
   __syncthreads();
 
-  // ---- 3. flush the tile's non-zero cells to the fine grid
+  // ---- 3. flush the tile's non-zero cells to the fine grid (even lanes the real and odd lanes the imaginary parts, whole
+  // lines per wave: 1451 us where this takes 1345; 8M clustered points, 128^3 modes)
   cplx<float>* fT = fw + (int64_t)tr * a.grid_cells;
-  for (int cell = tid; cell < TC; cell += kW3Threads) {
+  TileWalk<3> walk(tid, kW3Threads, T0, T1);
+  for (int cell = tid; cell < TC; cell += kW3Threads, walk.next()) {
     long long ir, ii;
     if constexpr (PK) {
       unpack_re_im(tile[cell], ir, ii);
@@ -344,7 +346,7 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
     if (finite && ir == 0 && ii == 0) continue;
     const float vr = finite ? (float)((double)ir * inv_scale) : NAN;
     const float vi = finite ? (float)((double)ii * inv_scale) : NAN;
-    const int64_t gi = tile_cell_to_global<3>(cell, a.tile, org, a.nf);
+    const int64_t gi = walk.at(org, a.nf);
     atomic_add_global(&fT[gi].re, vr);
     atomic_add_global(&fT[gi].im, vi);
   }
