@@ -4,7 +4,7 @@
 // Contract: perm == argsort(key, stable) and bin_start == [0, cumsum(bincount(key))],
 // where key = sum_d (floor(xs_d) div bs_d) * prod_{e<d} nb_e and xs is the FP64 fold.
 //
-// Counting sort, all integer work, in three launches (five above 1024 bins, see B):
+// Counting sort, all integer work, in three launches (four above 1024 bins, see B):
 //   A  k_keys: one block per chunk of points folds each point once, stores its
 //      key and counts the keys in LDS (per-lane integer atomics); the block writes
 //      its row of the histogram H[chunk][bin] (coalesced) and adds the row into
@@ -12,8 +12,9 @@
 //   B  k_seg_scan (one block): S -> exclusive prefixes over the segments (P) and
 //      bin totals, the totals -> bin_start and, per bin, the first subproblem
 //      (sub_start); S is cleared for the next sort.  Above 1024 bins the prefixes run
-//      one thread per bin (k_seg_prefix), the bin scan in one block (k_bin_scan), and
-//      k_row_offsets turns every histogram row into first output slots.
+//      one thread per bin (k_seg_prefix, which also adds up each block's bins), and
+//      k_row_offsets finishes the bin scan (a block: the sums of the blocks before it and
+//      its own 256 bins) and turns every histogram row into first output slots.
 //   C  k_scatter: each block first fills its share of the subproblem descriptors
 //      {bin, first sorted slot, count} (bins split into <= maxsub points) used by
 //      the tiled spread/interp kernels; then the W waves of a chunk count their
@@ -110,7 +111,8 @@ __device__ __forceinline__ int block_excl_scan(int v, int& total) {
 struct ScanArgs {
   int32_t* H;          // [NB][nbins] chunk histograms
   int32_t* S;          // [nseg][nbins] segment sums (zero between sorts)
-  int32_t* P;          // [nseg][nbins] exclusive prefixes over the segments
+  int32_t* P;          // [nseg][nbins] exclusive prefixes over the segments (above 1024 bins row 0: bin totals)
+  int32_t* blk;        // above 1024 bins: points and subproblems of every 256 bins (in subprob's memory)
   int32_t* bin_start;  // [nbins + 1]
   int32_t* sub_start;  // [nbins + 1]
   int32_t* nsub;
@@ -119,8 +121,8 @@ struct ScanArgs {
   int rows_are_offsets;  // H already holds first output slots (k_row_offsets ran)
 };
 
-// S -> P for bin b (exclusive over the segments, S cleared); the bin total into bin_start[b]
-__device__ __forceinline__ void seg_prefix_bin(const ScanArgs& sa, int b) {
+// S -> P for bin b (exclusive over the segments, S cleared); returns the bin total
+__device__ __forceinline__ int seg_prefix_bin(const ScanArgs& sa, int b) {
   constexpr int kG = 16;  // segment sums loaded together (independent loads in flight)
   int run = 0;
   for (int g0 = 0; g0 < sa.nseg; g0 += kG) {
@@ -137,12 +139,12 @@ __device__ __forceinline__ void seg_prefix_bin(const ScanArgs& sa, int b) {
       }
     }
   }
-  sa.bin_start[b] = run;
+  return run;
 }
 
 // one block: bin totals (in bin_start) -> exclusive scan = bin_start; subproblems per bin ->
-// sub_start; bin_start[nbins] = M; nsub.  Each thread takes a run of consecutive bins (16 at
-// 16384 bins and 1024 threads): its sums, one block scan, then its run written out.
+// sub_start; bin_start[nbins] = M; nsub.  Each thread takes a run of consecutive bins (one, at up
+// to 1024 bins): its sums, one block scan, then its run written out.
 __device__ __forceinline__ void bin_scan(const ScanArgs& sa) {
   const int per = (sa.nbins + (int)blockDim.x - 1) / (int)blockDim.x;
   const int b0 = (int)threadIdx.x * per, b1 = min(b0 + per, sa.nbins);
@@ -173,7 +175,7 @@ __device__ __forceinline__ void bin_scan(const ScanArgs& sa) {
 
 // few bins: the segment prefixes and the bin scan in one block
 __global__ void __launch_bounds__(1024) k_seg_scan(ScanArgs sa) {
-  for (int b = threadIdx.x; b < sa.nbins; b += blockDim.x) seg_prefix_bin(sa, b);
+  for (int b = threadIdx.x; b < sa.nbins; b += blockDim.x) sa.bin_start[b] = seg_prefix_bin(sa, b);
   __syncthreads();
   bin_scan(sa);
 }
@@ -181,23 +183,57 @@ __global__ void __launch_bounds__(1024) k_seg_scan(ScanArgs sa) {
 // many bins: segment prefixes one thread per bin, then the bin scan in one block, then the
 // chunk rows of the histogram turned into first output slots, H[r][b] -> slot of (bin b,
 // chunk r), so that a k_scatter block reads one offset per bin
+// Many bins.  The bin scan is spread over the blocks of the two kernels around it: one block that scanned all bins by
+// itself, 64 bytes apart per lane and two divisions a bin, took 28.6 us at 16384 bins.
 __global__ void __launch_bounds__(256) k_seg_prefix(ScanArgs sa) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b < sa.nbins) seg_prefix_bin(sa, b);
+  int c = 0;
+  if (b < sa.nbins) sa.P[b] = c = seg_prefix_bin(sa, b);
+  int total, total_sub;
+  (void)block_excl_scan(c, total);
+  (void)block_excl_scan((c + sa.maxsub - 1) / sa.maxsub, total_sub);
+  if (threadIdx.x == 0) {
+    sa.blk[2 * blockIdx.x] = total;
+    sa.blk[2 * blockIdx.x + 1] = total_sub;
+  }
 }
-
-__global__ void __launch_bounds__(1024) k_bin_scan(ScanArgs sa) { bin_scan(sa); }
 
 __global__ void __launch_bounds__(256) k_row_offsets(ScanArgs sa) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   const int seg = blockIdx.y;
+  // bins before this block's, then its own
+  int before = 0, base, total;
+  for (int i = threadIdx.x; i < (int)blockIdx.x; i += blockDim.x) before += sa.blk[2 * i];
+  (void)block_excl_scan(before, base);
+  const int c = b < sa.nbins ? sa.P[b] : 0;
+  const int start = base + block_excl_scan(c, total);
+  if (seg == 0) {
+    int before_sub = 0, base_sub, total_sub;
+    for (int i = threadIdx.x; i < (int)blockIdx.x; i += blockDim.x) before_sub += sa.blk[2 * i + 1];
+    (void)block_excl_scan(before_sub, base_sub);
+    const int nsb = (c + sa.maxsub - 1) / sa.maxsub;
+    const int sub = base_sub + block_excl_scan(nsb, total_sub);
+    if (b < sa.nbins) {
+      sa.bin_start[b] = start;
+      sa.sub_start[b] = sub;
+    }
+    if (b == sa.nbins - 1) {
+      sa.bin_start[sa.nbins] = sa.M;
+      sa.sub_start[sa.nbins] = sub + nsb;
+      *sa.nsub = min(sub + nsb, sa.max_subprob);
+    }
+  }
   if (b >= sa.nbins) return;
-  const int r0 = seg * kRowSeg, r1 = min(sa.NB, r0 + kRowSeg);
-  int run = sa.bin_start[b] + sa.P[(int64_t)seg * sa.nbins + b];
-  for (int r = r0; r < r1; ++r) {
-    const int t = sa.H[(int64_t)r * sa.nbins + b];
-    sa.H[(int64_t)r * sa.nbins + b] = run;
-    run += t;
+  const int r0 = seg * kRowSeg, nr = min(sa.NB - r0, kRowSeg);
+  int32_t* const h = sa.H + (int64_t)r0 * sa.nbins + b;
+  int t[kRowSeg];  // the segment's rows, all loads in flight
+#pragma unroll
+  for (int r = 0; r < kRowSeg; ++r) t[r] = r < nr ? h[(int64_t)r * sa.nbins] : 0;
+  int run = start + (seg > 0 ? sa.P[(int64_t)seg * sa.nbins + b] : 0);
+#pragma unroll
+  for (int r = 0; r < kRowSeg; ++r) {
+    if (r < nr) h[(int64_t)r * sa.nbins] = run;
+    run += t[r];
   }
 }
 
@@ -573,6 +609,7 @@ void launch_sort_passes(const KeyArgs& ka, PointSet& ps, int nbins, int W, int S
   sa.H = ps.hist;
   sa.S = ps.scan_sum;
   sa.P = ps.scan_part;
+  sa.blk = reinterpret_cast<int32_t*>(ps.subprob);  // the scatter fills the descriptors after the scan
   sa.bin_start = ps.bin_start;
   sa.sub_start = ps.sub_start;
   sa.nsub = ps.nsub;
@@ -589,7 +626,6 @@ void launch_sort_passes(const KeyArgs& ka, PointSet& ps, int nbins, int W, int S
   hipLaunchKernelGGL((k_keys<CT, D>), dim3(ps.NB), dim3(1024), lds_keys, s, ka, ps.M, CH, nbins, ps.keys, sa);
   if (sa.rows_are_offsets) {
     hipLaunchKernelGGL(k_seg_prefix, dim3((nbins + 255) / 256), dim3(256), 0, s, sa);
-    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, s, sa);
     hipLaunchKernelGGL(k_row_offsets, dim3((nbins + 255) / 256, sa.nseg), dim3(256), 0, s, sa);
   } else {
     hipLaunchKernelGGL(k_seg_scan, dim3(1), dim3(1024), 0, s, sa);

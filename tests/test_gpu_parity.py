@@ -92,6 +92,16 @@ def test_bin_sort_ragged_sizes(rng, M, kind):
     _check_sort([rng.uniform(-np.pi, np.pi, M) for _ in range(2)], (64, 48), kind)
 
 
+@pytest.mark.parametrize("n_modes", [(60, 66, 50), (70, 66, 50), (125, 125, 120)])
+@pytest.mark.parametrize("M", [1, 300, 70001])
+def test_bin_sort_many_bins_ragged(rng, n_modes, M):
+    """Above 1024 bins, not whole blocks of 256: first slots from the block sums; a third of the points in the last bin."""
+    coords = [rng.uniform(-np.pi, np.pi, M) for _ in range(3)]
+    for x in coords:
+        x[: M // 3] = -1e-3 * rng.uniform(0.1, 1.0, M // 3)
+    _check_sort(coords, n_modes)
+
+
 def test_bin_sort_one_bin_many_points(rng):
     """every point in one bin (the one-comparison ranking path), plus a second bin at the end."""
     M = 100_000
