@@ -28,6 +28,9 @@
 //      imaginary low, scale 2^(30 - e) with 2^e above S, which bounds every window value and
 //      every final tile value; the words add modulo 2^64 and only final sums must fit 31 bits);
 //   3. flush: the tile's non-zero cells go to the fine grid with FP32 global atomics.
+// What bounds it: the flush's global atomics, 141M of them for 8M clustered points with 128^3 modes (430 us at the 330 G/s
+// that coalesced FP32 atomics reach), and one block per CU, whose phases do not overlap: 1331 us there.  (Zero window
+// cells skipped in the flush to the tile: 1365.  The tile's words read four at a time in the last flush: 1340.)
 // The per-wave LDS blocks (weight rows, meta, strengths) are whole multiples of 16 bytes: an
 // odd-sized block misaligns the int4 meta reads of every other wave (1.70 -> 1.93 ms on 8M
 // clustered points).
@@ -102,7 +105,8 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
   float2* cval = reinterpret_cast<float2*>(meta + kW3K);      // scaled strengths
   int org[3];
   tile_origin<3>(sd, a.bs, a.nb, NS / 2, org);
-  for (int e = tid; e < (PK ? 1 : 2) * TC; e += kW3Threads) tile[e] = 0;
+  // bins are whole sub-bins, so a tile has an even number of words
+  for (int e = tid; e < (PK ? 1 : 2) * TC / 2; e += kW3Threads) reinterpret_cast<uint4*>(tile)[e] = make_uint4(0u, 0u, 0u, 0u);
   for (int e = lane; e < kW3RowF; e += 64)
     if (e % kWinRow < 16 - NS || e % kWinRow == 16 || e >= kW3K * kWinRow) {
       rowx[e] = 0.0f;
@@ -160,27 +164,28 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
     ssum[wave] = mysum;
   }
   __syncthreads();
-  if (tid < 16) {
-    int c = 0;
-    for (int e = 0; e < kW3Ppt * W; ++e) c += wcnt[e * 16 + tid];
-    cnt[tid] = c;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int acc = 0;
-    for (int s = 0; s < 16; ++s) {
-      start[s] = acc;
-      acc += (cnt[s] + kW3K - 1) & ~(kW3K - 1);
-    }
-    start[16] = acc;
-  }
-  __syncthreads();
-  if (tid < 16) {
-    int run = start[tid];
+  if (tid < 16) {  // counts per sub-bin, padded starts (16 lanes of one wave), first slot of every (pass, wave) run
+    int v[kW3Ppt * W], c = 0;
+#pragma unroll
     for (int e = 0; e < kW3Ppt * W; ++e) {
-      const int v = wcnt[e * 16 + tid];
+      v[e] = wcnt[e * 16 + tid];
+      c += v[e];
+    }
+    const int padded = (c + kW3K - 1) & ~(kW3K - 1);
+    int incl = padded;
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) {
+      const int t = __shfl_up(incl, off, 16);
+      if (tid >= off) incl += t;
+    }
+    cnt[tid] = c;
+    start[tid] = incl - padded;
+    if (tid == 15) start[16] = incl;
+    int run = incl - padded;
+#pragma unroll
+    for (int e = 0; e < kW3Ppt * W; ++e) {
       wcnt[e * 16 + tid] = (unsigned short)run;
-      run += v;
+      run += v[e];
     }
   }
   __syncthreads();
@@ -332,7 +337,7 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
   __syncthreads();
 
   // ---- 3. flush the tile's non-zero cells to the fine grid (even lanes the real and odd lanes the imaginary parts, whole
-  // lines per wave: 1451 us where this takes 1345; 8M clustered points, 128^3 modes)
+  // lines per wave: 1451 us where one lane per cell took 1345; 8M clustered points, 128^3 modes)
   cplx<float>* fT = fw + (int64_t)tr * a.grid_cells;
   TileWalk<3> walk(tid, kW3Threads, T0, T1);
   for (int cell = tid; cell < TC; cell += kW3Threads, walk.next()) {
