@@ -156,7 +156,7 @@ SortSizes sort_sizes(int64_t M, const Geometry& g, const SortTuning& tune, int r
 // want_slot (2D, 3D): also write the inverse permutation, and size the packed records for
 // n_trans transforms (n_trans 0: left to the first spread)
 hipError_t pointset_sort(PointSet& ps, const Geometry& g, const SortTuning& tune, hipStream_t s, std::string& err,
-                         int rec_kind = 0, int sub_sb = 0, bool want_slot = false, int64_t n_trans = 1);
+                         int rec_kind = 0, int sub_sb = 0, bool want_slot = false, int64_t n_trans = 1, bool reserve_only = false);
 // packed[t][slot[i]] = {x word, y word, c[t][i]} of a 2D point set sorted with want_slot (FP32
 // strengths; a non-finite coordinate makes its strength NaN); the same launch clears
 // zero_bytes (a multiple of 16) at zero, when given

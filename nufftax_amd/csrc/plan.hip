@@ -479,8 +479,8 @@ int check_plan(nufftx_plan p) {
   return NUFFTX_OK;
 }
 
-// interp: the point set is interpolated to (type 2, grid operators, type-3 targets).
-int sort_points(nufftx_plan p, PointSet& ps, const Geometry& g, bool interp, bool spread) {
+// interp: the point set is interpolated to (type 2, grid operators, type-3 targets).  reserve_only: the buffers, no sort.
+int sort_points(nufftx_plan p, PointSet& ps, const Geometry& g, bool interp, bool spread, bool reserve_only = false) {
   std::string err;
   SortTuning tune = p->tune;
   // point sets that the window kernels spread or interpolate get subproblems of up to 4096
@@ -500,7 +500,7 @@ int sort_points(nufftx_plan p, PointSet& ps, const Geometry& g, bool interp, boo
   const bool slot = win2d_geometry(g, p->prec, tune.maxsub) ||
                     (spread && win_spread_enabled() && win3d_geometry(g, p->prec, tune.maxsub));
   hipError_t e = pointset_sort(ps, g, tune, p->stream, err, rec_kind, subsort ? 16 - g.ns : 0, slot,
-                               spread ? p->n_trans : 0);
+                               spread ? p->n_trans : 0, reserve_only);
   if (e != hipSuccess) {
     if (!err.empty()) return fail(NUFFTX_ERR_INVALID_ARG, err);
     return fail(NUFFTX_ERR_HIP, std::string("bin-sort: ") + hipGetErrorString(e));
@@ -518,14 +518,21 @@ int sort_points(nufftx_plan p, PointSet& ps, const Geometry& g, bool interp, boo
     if (grow_buffer(ps.cmax, ps.cap_cmax, p->n_trans * (1 + std::max<int64_t>(nb, 1)), ps.retired) != hipSuccess)
       return fail(NUFFTX_ERR_ALLOC, "strength bound buffer");
   }
-  ps.sorted = true;
+  ps.sorted = !reserve_only;
   return NUFFTX_OK;
 }
 
-// Sorts a point set of setpts that has not been sorted yet (1D: direct1d.hip needs no sort).
-int need_sorted(nufftx_plan p, bool inner) {
+// Sorts a point set of setpts that has not been sorted yet (1D: direct1d.hip needs no sort).  A sort that is captured into a
+// graph runs with its replays only, so the points stay unsorted for every other call.
+int need_sorted(nufftx_plan p, bool inner, bool reserve_only = false) {
   PointSet& ps = inner ? p->pt : p->ps;
-  return ps.sorted ? NUFFTX_OK : sort_points(p, ps, inner ? p->gi : p->g, inner || p->type != 1, !inner && p->type != 2);
+  if (ps.sorted) return NUFFTX_OK;
+  const int r = sort_points(p, ps, inner ? p->gi : p->g, inner || p->type != 1, !inner && p->type != 2, reserve_only);
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (ps.sorted && (inner ? p->gi : p->g).dim == 1 && hipStreamIsCapturing(p->stream, &st) == hipSuccess &&
+      st != hipStreamCaptureStatusNone)
+    ps.sorted = false;
+  return r;
 }
 
 // setpts: sort now, unless neither the forward use nor (1D) anything else needs it yet
@@ -533,8 +540,9 @@ int set_points(nufftx_plan p, bool inner) {
   const Geometry& g = inner ? p->gi : p->g;
   (inner ? p->pt : p->ps).sorted = false;
   const bool spreads = !inner && (p->type == 1 || p->type == 3);
-  if (g.dim == 1 && interp1d_direct(g) && (!spreads || spread1d_direct(g))) return NUFFTX_OK;
-  return need_sorted(p, inner);
+  // the buffers of a later sort are sized here, so that a captured call allocates nothing
+  const bool later = g.dim == 1 && interp1d_direct(g) && (!spreads || spread1d_direct(g));
+  return need_sorted(p, inner, later);
 }
 
 // before a spread from the plan's points, and before a gather of coordinate gradients

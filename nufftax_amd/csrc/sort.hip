@@ -703,7 +703,7 @@ SortSizes sort_sizes(int64_t M, const Geometry& g, const SortTuning& tune, int r
 }
 
 hipError_t pointset_sort(PointSet& ps, const Geometry& g, const SortTuning& tune, hipStream_t s, std::string& err,
-                         int rec_kind, int sub_sb, bool want_slot, int64_t n_trans) {
+                         int rec_kind, int sub_sb, bool want_slot, int64_t n_trans, bool reserve_only) {
   hipError_t e;
   const int nbins = g.nbins;
   if ((int64_t)nbins * sizeof(int32_t) > 65536) {
@@ -761,6 +761,7 @@ hipError_t pointset_sort(PointSet& ps, const Geometry& g, const SortTuning& tune
     hipLaunchKernelGGL(k_zero_i32, dim3(nz), dim3(256), 0, s, ps.scan_sum, ps.cap_sum);
   }
   ps.max_subprob = (int)max_sub;
+  if (reserve_only) return hipGetLastError();
 
   if (M == 0) {
     hipLaunchKernelGGL(k_empty_sort, dim3(1), dim3(256), 0, s, nbins, ps.bin_start, ps.nsub);

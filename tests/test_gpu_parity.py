@@ -1170,3 +1170,43 @@ def test_direct1d_sorts_when_asked(rng):
     ref_perm, ref_off = R.bin_sort(keys, nbins)
     np.testing.assert_array_equal(_np(perm).astype(np.int64), ref_perm)
     np.testing.assert_array_equal(_np(bst).astype(np.int64), ref_off)
+
+
+def test_direct1d_sort_under_capture(rng):
+    """A 1D plan's sort, put off by setpts, captured with the coordinate gradient that asks for it: an eager gradient before
+    the first replay and every replay equal the gradient of another plan with the same points."""
+    from nufftax_amd._plan import F32, Plan
+
+    M, nm = 5000, 300
+    dev = torch.device(DEV, 0)
+    x0, x1 = (_t(rng.uniform(-np.pi, np.pi, M).astype(np.float32)) for _ in range(2))
+    c = _t((rng.standard_normal(M) + 1j * rng.standard_normal(M)).astype(np.complex64))
+    g = _t((rng.standard_normal(nm) + 1j * rng.standard_normal(nm)).astype(np.complex64))
+    new = lambda: (torch.zeros(M, dtype=torch.complex64, device=DEV), torch.zeros(M, device=DEV))  # noqa: E731
+    other = Plan.transform(1, 1, (nm,), 1, 1e-6, 1, 2.0, F32, 0, dev)
+    other.setpts([x1])
+    want = new()
+    other.vjp(c, g, want[0], [want[1]])
+    plan = Plan.transform(1, 1, (nm,), 1, 1e-6, 1, 2.0, F32, 0, dev)
+    warm, eager, got = new(), new(), new()
+    plan.setpts([x0])
+    plan.vjp(c, g, warm[0], [warm[1]])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        plan.setpts([x1])
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            plan.vjp(c, g, got[0], [got[1]])
+        plan.vjp(c, g, eager[0], [eager[1]])
+        torch.cuda.synchronize()
+        for _ in range(3):
+            for t in got:
+                t.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            for a, b in zip(got, want):
+                assert R.rel_l2(_np(a), _np(b)) < 2e-6
+    for a, b in zip(eager, want):
+        assert R.rel_l2(_np(a), _np(b)) < 2e-6
