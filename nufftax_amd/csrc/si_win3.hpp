@@ -13,8 +13,8 @@
 // which no support reaches, are never flushed) and 4 in z.  Bins must be whole numbers of
 // sub-bins (at most 16 per bin); the 3D sort's bins of 16 x 8 x 8 or 16 x 16 x 8 cells are.
 //
-// Block = one subproblem (<= 2048 points of one bin), 8 waves:
-//   1. order: as in the 2D kernel (four points per thread), sub-bins padded to multiples of
+// Block = one subproblem (<= 4096 points of one bin), 8 waves:
+//   1. order: as in the 2D kernel (eight points per thread), sub-bins padded to multiples of
 //      32 with zero-strength entries; the block also takes max(|re c|, |im c|) and
 //      S = sum_j max(|re c_j|, |im c_j|);
 //   2. accumulate: contiguous ranges of groups per wave; per group, the lanes evaluate the
@@ -28,8 +28,11 @@
 //      imaginary low, scale 2^(30 - e) with 2^e above S, which bounds every window value and
 //      every final tile value; the words add modulo 2^64 and only final sums must fit 31 bits);
 //   3. flush: the tile's non-zero cells go to the fine grid with FP32 global atomics.
-// What bounds it: the flush's global atomics, 141M of them for 8M clustered points with 128^3 modes (430 us at the 330 G/s
-// that coalesced FP32 atomics reach), and one block per CU, whose phases do not overlap: 1331 us there.  (Zero window
+// What bounds it: the flush's global atomics and one block per CU, whose phases do not overlap.  8M clustered points with
+// 128^3 modes in subproblems of 2048: 141M atomics (430 us at the 330 G/s that coalesced FP32 atomics reach), 1331 us.
+// Subproblems of 4096, which the weights' blocks leave room for since the strengths moved into the meta words, flush the
+// dense bins half as often: the whole call 1960 -> 1913 us; taken where the points fill the chip with them (win3_maxsub).
+// (The counts of passes without points left out of the order phase: 2% slower.)  (Zero window
 // cells skipped in the flush to the tile: 1365.  The tile's words read four at a time in the last flush: 1340.)
 // The per-wave LDS blocks (weight rows, meta, strengths) are whole multiples of 16 bytes: an
 // odd-sized block misaligns the int4 meta reads of every other wave (1.70 -> 1.93 ms on 8M
@@ -41,8 +44,9 @@
 namespace nufftx {
 
 constexpr int kW3Threads = 512;                    // 8 waves per subproblem
-constexpr int kW3Ppt = 4;                          // points per thread while ordering
+constexpr int kW3Ppt = 8;                          // points per thread while ordering
 constexpr int kW3K = 32;                           // points per group
+constexpr int kW3Hold = 10;                        // groups summed in FP32 before they go to the exact tile
 constexpr int kW3SB = 8;                           // sub-bin side in x and y (support starts)
 constexpr int kW3SBZ = 4;                          // sub-bin side in z
 constexpr int kW3RowZ = 13;                        // z row stride (floats): 4 zeros, ns <= 8 weights, 1 zero
@@ -51,7 +55,7 @@ constexpr int kW3RowZ = 13;                        // z row stride (floats): 4 z
 // strengths stay aligned
 constexpr int kW3RowF = ((kW3K - 1) * kWinRow + 32 + 3) & ~3;   // x / y row block (floats)
 constexpr int kW3RowZF = ((kW3K - 1) * kW3RowZ + 16 + 3) & ~3;  // z row block (floats)
-constexpr int kW3WaveF = 2 * kW3RowF + kW3RowZF + 4 * kW3K + 2 * kW3K;  // + meta int4 + strength float2
+constexpr int kW3WaveF = 2 * kW3RowF + kW3RowZF + 4 * kW3K;  // + meta int4
 static_assert(kW3RowF % 4 == 0 && kW3RowZF % 4 == 0 && kW3WaveF % 4 == 0, "16-byte aligned per-wave blocks");
 static_assert(kW3Threads * kW3Ppt == kWin3MaxSub, "win3d_geometry admits subproblems of up to kWin3MaxSub points");
 
@@ -101,8 +105,7 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
   float* rowx = lf + wof;
   float* rowy = rowx + kW3RowF;
   float* rowz = rowy + kW3RowF;
-  int4* meta = reinterpret_cast<int4*>(rowz + kW3RowZF);     // {y read index, x read index, z read index, -}
-  float2* cval = reinterpret_cast<float2*>(meta + kW3K);      // scaled strengths
+  int4* meta = reinterpret_cast<int4*>(rowz + kW3RowZF);  // {read indices y | x << 16, z; scaled strength}
   int org[3];
   tile_origin<3>(sd, a.bs, a.nb, NS / 2, org);
   // bins are whole sub-bins, so a tile has an even number of words
@@ -235,7 +238,7 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
   }
   int s = 0;
   while (s < 15 && start[s + 1] <= kW3K * g0) ++s;
-  int next = start[s + 1];
+  int next = start[s + 1], held = 0;
   auto flush = [&](int sbin) {
     const int sx = sbin % nsx, sy = (sbin / nsx) % nsy, sz = sbin / (nsx * nsy);
     const int x = sx * kW3SB + i;
@@ -267,18 +270,18 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
   float2 cv;
   fetch(g0, p, cv);
   for (int g = g0; g < g1 && finite; ++g) {
-    if (kW3K * g >= next) {
+    if (kW3K * g >= next || held == kW3Hold) {
+      held = 0;
       flush(s);
 #pragma unroll
       for (int z = 0; z < WZ; ++z) {
         acc_re[z] = win_f4{0.f, 0.f, 0.f, 0.f};
         acc_im[z] = win_f4{0.f, 0.f, 0.f, 0.f};
       }
-      do {
-        ++s;
-      } while (s < 15 && start[s + 1] <= kW3K * g);
+      while (s < 15 && start[s + 1] <= kW3K * g) ++s;
       next = start[s + 1];
     }
+    ++held;
     // -- kernel weights: lanes 0-31 x, 32-63 y (all ns); then z, ns/2 per lane
     {
       const unsigned wd = shi ? p.y : p.x;
@@ -295,8 +298,8 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
         const int lx = (int)(p.x >> 25), ly = (int)(p.y >> 25), lz = (int)(p.z >> 25);
         const int ox = lx - min(lx / kW3SB, nsx - 1) * kW3SB, oy = ly - min(ly / kW3SB, nsy - 1) * kW3SB;
         const int oz = lz - min(lz / kW3SBZ, nsz - 1) * kW3SBZ;
-        meta[sq] = make_int4(ry0 + kWinRow * sq - oy, rx0 + kWinRow * sq - ox, rz0 + kW3RowZ * sq - oz, 0);
-        cval[sq] = make_float2(ldexpf(cv.x, ke), ldexpf(cv.y, ke));
+        meta[sq] = make_int4((ry0 + kWinRow * sq - oy) | (rx0 + kWinRow * sq - ox) << 16, rz0 + kW3RowZ * sq - oz,
+                             __float_as_int(ldexpf(cv.x, ke)), __float_as_int(ldexpf(cv.y, ke)));
       }
     }
     fetch(g + 1, p, cv);
@@ -307,12 +310,11 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int4 mt = meta[8 * kq + e];
-      const float2 c2 = cval[8 * kq + e];
-      wy[e] = lf[mt.x + i];
-      wx[e] = lf[mt.y + i];
-      zb[e] = mt.z;
-      cre[e] = c2.x;
-      cim[e] = c2.y;
+      wy[e] = lf[(mt.x & 0xFFFF) + i];
+      wx[e] = lf[((unsigned)mt.x >> 16) + i];
+      zb[e] = mt.y;
+      cre[e] = __int_as_float(mt.z);
+      cim[e] = __int_as_float(mt.w);
     }
     wh_h8 arh, arl, aih, ail;
     split_prod_f16(cre, wy, arh, arl);

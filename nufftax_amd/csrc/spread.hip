@@ -150,7 +150,7 @@ bool spread_win(const GridOpArgs& ga, const void* c, void* fw, hipStream_t s, hi
     }
     const bool exact = win_exact_tiles();
     const size_t lds = exact ? win_spread_lds<NS, false>(ps.maxsub) : win_spread_lds<NS, true>(ps.maxsub);
-    if (lds + 2048 > (size_t)lds_device_max_bytes()) return false;
+    if (lds + 2304 > (size_t)lds_device_max_bytes()) return false;
     if (ga.zero_out && !fused_zero && (err = launch_zero(fw, grid_bytes, s)) != hipSuccess) return true;
     if ((err = pointset_pack2d(ps, *ga.g, c, ga.n_trans, s, zero, zero_bytes)) != hipSuccess) return true;
     auto kern = exact ? k_spread_win2d<NS, false> : k_spread_win2d<NS, true>;
@@ -178,13 +178,13 @@ bool spread_win3d(const GridOpArgs& ga, const void* c, void* fw, hipStream_t s, 
   PointSet& ps = const_cast<PointSet&>(*ga.ps);
   if (!win3d_geometry(*ga.g, ga.prec, ps.maxsub) || !ps.has_slot || !win_spread_enabled()) return false;
   SIArgs<float> a = make_si_args<float>(ga);
-  // the static LDS (ordering counters) is below 2 KB
+  // the static LDS (ordering counters) is below 2304 bytes
   const size_t lds_exact = w3_spread_lds<false>(ga.g->tile_cells, ps.maxsub);
   const size_t lds_packed = w3_spread_lds<true>(ga.g->tile_cells, ps.maxsub);
   const char* pe = std::getenv("NUFFTX_WIN3_PACKED");
-  const bool exact = lds_exact + 2048 <= (size_t)lds_device_max_bytes() && !(pe && pe[0] == '1');
+  const bool exact = lds_exact + 2304 <= (size_t)lds_device_max_bytes() && !(pe && pe[0] == '1');
   const size_t lds = exact ? lds_exact : lds_packed;
-  if (lds + 2048 > (size_t)lds_device_max_bytes()) return false;
+  if (lds + 2304 > (size_t)lds_device_max_bytes()) return false;
   const int64_t grid_bytes = ga.n_trans * ga.g->grid_cells() * (int64_t)sizeof(cplx<float>);
   const bool fused_zero = ga.zero_out && grid_bytes % 16 == 0;
   if (ga.zero_out && !fused_zero && (err = launch_zero(fw, grid_bytes, s)) != hipSuccess) return true;
