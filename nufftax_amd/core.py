@@ -44,6 +44,7 @@ from ._lib import F32, F64, check, lib, ptr
 from ._plan import _stream_handle, grid_plan
 from .params import KernelParams, compute_kernel_params
 from .transforms import _run
+from .utils import dense
 
 __all__ = [
     "es_kernel", "es_kernel_with_derivative", "compute_kernel_params", "kernel_fourier_series", "KernelParams",
@@ -194,7 +195,7 @@ def _norm_coords(coords, rdt, dev):
         x = x.detach().to(device=dev, dtype=rdt)
         if x.ndim != 1 or x.shape[0] != M:
             raise ValueError(f"coordinate arrays must have shape ({M},), got {tuple(x.shape)}")
-        out.append(x.contiguous())
+        out.append(dense(x))
     return out, M
 
 
@@ -212,7 +213,7 @@ def _raw_spread(ctx: _GridCtx, coords, c):
     plan = _plan_for(ctx, n_trans, prec, dev)
     with plan.lock:
         plan.setpts(xs)
-        plan.spread(c.contiguous(), fw)
+        plan.spread(dense(c), fw)
     return fw
 
 
@@ -228,7 +229,7 @@ def _raw_interp(ctx: _GridCtx, coords, fw):
     plan = _plan_for(ctx, n_trans, prec, dev)
     with plan.lock:
         plan.setpts(xs)
-        plan.interp(fw.contiguous(), c)
+        plan.interp(dense(fw), c)
     return c
 
 
@@ -244,7 +245,7 @@ def _raw_coord_grad(ctx: _GridCtx, coords, G, P):
     plan = _plan_for(ctx, n_trans, prec, dev)
     with plan.lock:
         plan.setpts(xs)
-        plan.gather_grad(G.contiguous(), P.to(cdt).contiguous(), None, grads)
+        plan.gather_grad(dense(G), dense(P.to(cdt)), None, grads)
     return grads
 
 
@@ -393,11 +394,11 @@ def _deconvolve(direction, arr, phihats, dim, n_modes, nf, modeord):
             raise ValueError(f"n_modes {n_modes} must be in [1, nf] for nf {nf}")
     ph = []
     for d in range(dim):
-        p = _to_dev(phihats[d], dev).to(rdt).contiguous()
+        p = dense(_to_dev(phihats[d], dev).to(rdt))
         if p.ndim != 1 or p.shape[0] < n_modes[d] // 2 + 1:
             raise ValueError(f"phihat for axis {d} must have at least {n_modes[d] // 2 + 1} entries")
         ph.append(p)
-    src = a.reshape((n_trans,) + inner).contiguous()
+    src = dense(a.reshape((n_trans,) + inner))
     out = torch.empty((n_trans,) + outer, dtype=cdt, device=dev)
     nm = (ctypes.c_int64 * 3)(*(list(n_modes) + [1] * (3 - dim)))
     nfa = (ctypes.c_int64 * 3)(*(list(nf) + [1] * (3 - dim)))

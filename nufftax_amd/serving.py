@@ -47,6 +47,7 @@ import torch
 from . import _lib
 from ._plan import F32, F64, Plan
 from .params import compute_grid_size, compute_kernel_params
+from .utils import dense
 
 __all__ = ["NufftServer", "ServeRequest", "latency_stats", "request_bytes"]
 
@@ -325,14 +326,14 @@ class NufftServer:
             _, dim, n_modes, _, _, prec = sig
             cdt = torch.complex128 if prec == F64 else torch.complex64
             rdt = torch.float64 if prec == F64 else torch.float32
-            coords = [x if (x.dtype == rdt and x.is_contiguous()) else x.to(rdt).contiguous() for x in first.coords]
+            coords = [dense(x.to(rdt)) for x in first.coords]
             M = coords[0].shape[0]
             if kind == 1:
                 datas = [g.data.reshape(-1, M) for g in unit]
             else:
                 datas = [g.data.reshape((-1,) + tuple(reversed(n_modes))) for g in unit]
             sizes = [d.shape[0] for d in datas]
-            src = torch.cat(datas, 0).to(cdt).contiguous() if len(datas) > 1 else datas[0].to(cdt).contiguous()
+            src = dense((torch.cat(datas, 0) if len(datas) > 1 else datas[0]).to(cdt))
             n_trans = src.shape[0]
             k = used.get((sig, n_trans), 0)
             used[(sig, n_trans)] = k + 1

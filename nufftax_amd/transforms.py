@@ -36,6 +36,7 @@ from torch.autograd.function import once_differentiable
 
 from . import _lib
 from ._plan import F32, F64, transform_plan
+from .utils import dense
 
 __all__ = [
     "nufft1d1", "nufft2d1", "nufft3d1",
@@ -113,7 +114,7 @@ def _coords(coords, rdt, device, M):
             x = x.to(device=device, dtype=rdt)
         if x.ndim != 1 or x.shape[0] != M:
             raise ValueError(f"coordinate arrays must have shape ({M},), got {tuple(x.shape)}")
-        out.append(x.contiguous())
+        out.append(dense(x))
     return out
 
 
@@ -138,7 +139,7 @@ def _raw_type1(meta: _Meta, c: torch.Tensor, coords, isign=None, upsampfac=None)
     prec, cdt, rdt = _work_dtypes(c.dtype, meta.eps)
     dev = c.device
     xs = _coords(coords, rdt, dev, M)
-    cc = c.reshape(n_trans, M).to(cdt).contiguous()
+    cc = dense(c.reshape(n_trans, M).to(cdt))
     isign = meta.isign if isign is None else isign
     uf = meta.upsampfac if upsampfac is None else upsampfac
     out = torch.empty((n_trans,) + tuple(reversed(meta.n_modes)), dtype=cdt, device=dev)
@@ -158,7 +159,7 @@ def _raw_type2(meta: _Meta, f: torch.Tensor, coords, isign=None, upsampfac=None)
     prec, cdt, rdt = _work_dtypes(f.dtype, meta.eps)
     dev = f.device
     xs = _coords(coords, rdt, dev, M)
-    ff = f.reshape((n_trans,) + tuple(reversed(nm))).to(cdt).contiguous()
+    ff = dense(f.reshape((n_trans,) + tuple(reversed(nm))).to(cdt))
     isign = meta.isign if isign is None else isign
     uf = meta.upsampfac if upsampfac is None else upsampfac
     out = torch.empty((n_trans, M), dtype=cdt, device=dev)
@@ -179,7 +180,7 @@ def _raw_type3(meta: _Meta, c: torch.Tensor, coords, targets, isign=None):
     dev = c.device
     xs = _coords(coords, rdt, dev, M)
     ss = _coords(targets, rdt, dev, N)
-    cc = c.reshape(n_trans, M).to(cdt).contiguous()
+    cc = dense(c.reshape(n_trans, M).to(cdt))
     isign = meta.isign if isign is None else isign
     out = torch.empty((n_trans, N), dtype=cdt, device=dev)
     for s, e in _chunks(n_trans):
@@ -205,11 +206,11 @@ def _vjp_type12(kind, meta: _Meta, src, coords, g, need_src, need_coord):
         n_modes = tuple(reversed(src.shape[src.ndim - dim:]))
         src_shape2 = (-1,) + tuple(reversed(n_modes))
     n_trans = int(math.prod(lead)) if lead else 1
-    ss = src.reshape(src_shape2).to(cdt).contiguous()
+    ss = dense(src.reshape(src_shape2).to(cdt))
     if kind == 1:
-        gg = g.reshape((n_trans,) + tuple(reversed(n_modes))).to(cdt).contiguous()
+        gg = dense(g.reshape((n_trans,) + tuple(reversed(n_modes))).to(cdt))
     else:
-        gg = g.reshape(n_trans, M).to(cdt).contiguous()
+        gg = dense(g.reshape(n_trans, M).to(cdt))
     grad_src = torch.empty_like(ss) if need_src else None
     # one chunk writes the gradients themselves; several (more than MAX_TRANS transforms) add up
     one = 1 <= n_trans <= MAX_TRANS

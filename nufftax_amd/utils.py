@@ -3,6 +3,16 @@
 import torch
 
 
+def dense(x: torch.Tensor) -> torch.Tensor:
+    """x as a kernel reads it through its pointer: contiguous, and without the conjugate or negative
+    bit of a lazy view (``c.conj()`` and ``c.conj().imag`` share c's memory)."""
+    if x.is_conj():
+        x = x.resolve_conj()
+    if x.is_neg():
+        x = x.resolve_neg()
+    return x.contiguous()
+
+
 def to_complex(x: torch.Tensor) -> torch.Tensor:
     """(..., 2) real/imag -> complex (...)."""
     return torch.complex(x[..., 0], x[..., 1])

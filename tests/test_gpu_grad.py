@@ -292,3 +292,27 @@ def test_plan_vjp_writes_whole_gradients(rng, dim, M, n_trans, double):
     for d in range(dim):
         want = np.real(np.einsum("tj,tk,kj,k->j", cc, gg.conj(), E, 1j * ks[d].ravel(), optimize=True))
         assert R.rel_l2(_np(grads[d]), want) < 20 * eps
+
+
+def test_lazily_conjugated_inputs_and_cotangents(rng):
+    """c.conj() as strengths, and a loss that hands the backward a lazily conjugated cotangent, against the same values laid
+    out by .clone(): the library reads the values, not the memory that the view shares (bit-equal up to the order of the
+    spread's FP64 atomics)."""
+    import nufftax_amd as N
+
+    x = _t(rng.uniform(-np.pi, np.pi, 300))
+    c = _t(rng.standard_normal(300) + 1j * rng.standard_normal(300))
+    w = _t(rng.standard_normal(20) + 1j * rng.standard_normal(20))
+    lazy = c.conj()
+    assert lazy.is_conj()
+    got, want = N.nufft1d1(x, lazy, 20, eps=1e-9), N.nufft1d1(x, lazy.resolve_conj().clone(), 20, eps=1e-9)
+    assert R.rel_l2(_np(got), _np(want)) < 1e-12
+
+    def grads(lay_out):
+        cc, xx = c.clone().requires_grad_(True), x.clone().requires_grad_(True)
+        out = N.nufft1d1(xx, cc, 20, eps=1e-9)
+        cot = w.conj()
+        return torch.autograd.grad(out, [cc, xx], cot.resolve_conj().clone() if lay_out else cot)
+
+    for a, b in zip(grads(False), grads(True)):
+        assert R.rel_l2(_np(a), _np(b)) < 1e-12

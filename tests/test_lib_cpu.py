@@ -351,3 +351,66 @@ def test_autodiff_dispatch_predicate():
     torch.func.jvp(probe, (x,), (torch.ones(4),))
     torch.func.grad(lambda v: probe(v).sum())(x)
     assert seen == [True, True, True]
+
+
+class _RecordingPlan:
+    """Stands in for a plan and keeps the tensors whose pointers the library would be given."""
+
+    def __init__(self):
+        import threading
+
+        self.lock = threading.RLock()
+        self.seen = []
+
+    def _keep(self, *args):
+        for a in args:
+            for t in a if isinstance(a, (list, tuple)) else [a]:
+                if hasattr(t, "is_conj"):
+                    self.seen.append(t)
+
+    def run(self, coords, targets, c, f, isign):
+        self._keep(coords, targets, c, f)
+
+    setpts = spread = interp = vjp = gather_grad = execute = lambda self, *args, **kw: self._keep(*args)
+
+
+def test_lazy_views_reach_the_library_as_values(monkeypatch):
+    """A conjugated or negated tensor that shares another's memory is laid out before its pointer is taken: strengths, modes,
+    coordinates and cotangents of the transforms, the core operators and the server."""
+    import types
+
+    import torch
+
+    from nufftax_amd import core, serving, transforms as T
+
+    plan = _RecordingPlan()
+    monkeypatch.setattr(T, "transform_plan", lambda *a, **k: plan)
+    monkeypatch.setattr(core, "_plan_for", lambda *a, **k: plan)
+    z = torch.randn(6, dtype=torch.complex64)
+    c, x = z.conj(), z.conj().imag
+    f = torch.randn(4, 5, dtype=torch.complex64).conj()
+    assert c.is_conj() and x.is_neg() and f.is_conj()
+    m1, m2 = T._Meta(1, (8,), 1e-6, 1, 2.0, 2.0), T._Meta(2, (5, 4), 1e-6, 1, 2.0, 2.0)
+    g1 = torch.randn(8, dtype=torch.complex64).conj()
+    kp = core.compute_kernel_params(1e-6)
+    gctx = core._GridCtx(1, (32,), kp)
+    fw = torch.randn(1, 32, dtype=torch.complex64).conj()
+    server = types.SimpleNamespace(_plan=lambda *a: plan, device=torch.device("cpu"))
+    calls = [
+        (lambda: T._raw_type1(m1, c, [x]), [c, x]),
+        (lambda: T._raw_type2(m2, f, [x, x]), [f, x]),
+        (lambda: T._raw_type3(m1, c, [x], [x]), [c, x]),
+        (lambda: T._vjp_type12(1, m1, c, [x], g1, True, [True]), [c, g1, x]),
+        (lambda: T._vjp_type12(2, m2, f, [x, x], c, True, [True, True]), [f, c, x]),
+        (lambda: core._raw_spread(gctx, [x], c[None]), [c, x]),
+        (lambda: core._raw_interp(gctx, [x], fw), [fw, x]),
+        (lambda: core._raw_coord_grad(gctx, [x], fw, c[None]), [fw, c, x]),
+        (lambda: serving.NufftServer._launch(server, [[serving.ServeRequest(1, (x,), c, (8,), 1e-6, 1)]]), [c, x]),
+    ]
+    for call, inputs in calls:
+        plan.seen.clear()
+        call()
+        assert plan.seen and not any(t.is_conj() or t.is_neg() for t in plan.seen)
+        for want in inputs:
+            assert any(t.numel() == want.numel() and t.is_complex() == want.is_complex()
+                       and torch.equal(t.reshape(-1), want.reshape(-1)) for t in plan.seen)
