@@ -77,7 +77,7 @@ struct PointSet {
   int64_t cap_slot = 0, cap_packed = 0, cap_cs = 0;
   int64_t cap_recs = 0, cap_sub_off = 0, cap_cmax = 0;
   int64_t cap_M = 0, cap_keys = 0, cap_hist = 0, cap_part = 0, cap_bins = 0, cap_sub = 0, cap_sub_start = 0;
-  // 3D FP64 point sets spread by output regions (spread64.hip), per execute
+  // 3D FP64 point sets spread by output regions (spread64.hip), filled per execute
   double* tab64 = nullptr;       // M * 3 ns kernel weights in sorted order
   int4* start64 = nullptr;       // M support starts
   double2* cs64 = nullptr;       // n_trans * M strengths in sorted order
@@ -234,7 +234,8 @@ hipError_t launch_interp_grad(const GridOpArgs& a, const void* G, const void* P,
 constexpr int64_t kSpread64MinPoints = 2048;
 bool spread64_applicable(const Geometry& g, int prec, int64_t M);
 hipError_t spread64_reserve(PointSet& ps, const Geometry& g, int64_t n_trans);  // buffers for M points
-hipError_t launch_spread64(const GridOpArgs& a, const void* c, void* fw, hipStream_t s);
+bool spread64_reserved(const PointSet& ps, const Geometry& g, int64_t n_trans);
+hipError_t launch_spread64(const GridOpArgs& a, const void* c, void* fw, hipStream_t s);  // of a reserved point set
 
 // ---- direct1d.hip: 1D spreading (small grids) and interpolation (any grid) without a sort
 bool spread1d_direct(const Geometry& g);

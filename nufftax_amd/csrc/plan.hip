@@ -511,8 +511,10 @@ int sort_points(nufftx_plan p, PointSet& ps, const Geometry& g, bool interp, boo
     e = pointset_subsort(ps, g, p->stream);
     if (e != hipSuccess) return fail(NUFFTX_ERR_HIP, std::string("sub-bin sort: ") + hipGetErrorString(e));
   }
-  if (spread && spread64_applicable(g, p->prec, ps.M) && spread64_reserve(ps, g, p->n_trans) != hipSuccess)
-    return fail(NUFFTX_ERR_ALLOC, "FP64 spreading buffers");
+  // the region spread's buffers, for type 2 too (its vjp spreads), so that no later call allocates; the atomic kernels,
+  // which need none, take over where they cannot be had
+  if (&ps == &p->ps && spread64_applicable(g, p->prec, ps.M) && spread64_reserve(ps, g, p->n_trans) != hipSuccess)
+    (void)hipGetLastError();
   // the FP32 spreading kernels' strength bound (n_trans values and the per-block partial
   // maxima) is sized here, so that execute allocates nothing for a point set of this size
   if (p->prec == kF32) {

@@ -531,22 +531,27 @@ bool spread64_applicable(const Geometry& g, int prec, int64_t M) {
          M * 3 * g.ns * (int64_t)sizeof(double) <= kTabMaxBytes && z.tasks <= INT32_MAX;
 }
 
+// Buffers of a spread, the largest last: a set that cannot be had leaves the small ones only.
 hipError_t spread64_reserve(PointSet& ps, const Geometry& g, int64_t n_trans) {
   const Sizes64 z = sizes64(g, ps.M);
   hipError_t e;
-  if ((e = grow_buffer(ps.tab64, ps.cap_tab64, ps.M * 3 * g.ns, ps.retired)) != hipSuccess) return e;
-  if ((e = grow_buffer(ps.start64, ps.cap_start64, ps.M, ps.retired)) != hipSuccess) return e;
-  if ((e = grow_buffer(ps.cs64, ps.cap_cs64, ps.M * n_trans, ps.retired)) != hipSuccess) return e;
-  if ((e = grow_buffer(ps.bad64, ps.cap_bad64, ps.M * n_trans, ps.retired)) != hipSuccess) return e;
+  if ((e = grow_buffer(ps.heavy64, ps.cap_heavy64, z.regions + 4, ps.retired)) != hipSuccess) return e;
   if ((e = grow_buffer(ps.task64, ps.cap_task64, z.tasks, ps.retired)) != hipSuccess) return e;
-  return grow_buffer(ps.heavy64, ps.cap_heavy64, z.regions + 4, ps.retired);
+  if ((e = grow_buffer(ps.start64, ps.cap_start64, ps.M, ps.retired)) != hipSuccess) return e;
+  if ((e = grow_buffer(ps.bad64, ps.cap_bad64, ps.M * n_trans, ps.retired)) != hipSuccess) return e;
+  if ((e = grow_buffer(ps.cs64, ps.cap_cs64, ps.M * n_trans, ps.retired)) != hipSuccess) return e;
+  return grow_buffer(ps.tab64, ps.cap_tab64, ps.M * 3 * g.ns, ps.retired);
+}
+
+bool spread64_reserved(const PointSet& ps, const Geometry& g, int64_t n_trans) {
+  const Sizes64 z = sizes64(g, ps.M);
+  return ps.cap_heavy64 >= z.regions + 4 && ps.cap_task64 >= z.tasks && ps.cap_start64 >= ps.M &&
+         ps.cap_bad64 >= ps.M * n_trans && ps.cap_cs64 >= ps.M * n_trans && ps.cap_tab64 >= ps.M * 3 * g.ns;
 }
 
 hipError_t launch_spread64(const GridOpArgs& ga, const void* c, void* fw, hipStream_t s) {
-  PointSet& ps = const_cast<PointSet&>(*ga.ps);
+  const PointSet& ps = *ga.ps;
   const Geometry& g = *ga.g;
-  hipError_t e = spread64_reserve(ps, g, ga.n_trans);
-  if (e != hipSuccess) return e;
   const Sizes64 z = sizes64(g, ps.M);
   Reg64Args a;
   a.M = ps.M;

@@ -73,3 +73,55 @@ def test_spread_noalloc_rejects_sizes_above_its_limit():
     big = _lib.NOALLOC_MAX_POINTS + 1
     rc = L.nufftx_spread_noalloc(2, nfa, 8, 18.6, 1.0 / 16, 0, big, None, None, None, None, None, None)
     assert rc == 1 and b"NOALLOC_MAX_POINTS" in L.nufftx_last_error()
+
+
+def test_fp64_region_spread_allocates_at_setpts_only():
+    """The 3D FP64 region spread's buffers belong to setpts: spread_noalloc (5000 points, which a plan spreads by regions) and
+    the vjp of a type-2 plan make no device allocation, and that vjp can be captured without a call before."""
+    from nufftax_amd import _lib
+    from nufftax_amd._plan import F64, Plan, grid_plan
+
+    L = _lib.lib()
+    dev = torch.device(DEV, 0)
+    rng = np.random.default_rng(3)
+    M, nf, nm = 5000, (48, 40, 36), (20, 18, 16)
+    kp = R.compute_kernel_params(1e-12)
+    xs = [torch.as_tensor(rng.uniform(-np.pi, np.pi, M), device=DEV) for _ in range(3)]
+    cplx = lambda *s: torch.as_tensor(rng.standard_normal(s) + 1j * rng.standard_normal(s), device=DEV)  # noqa: E731
+    c, f, out, ref = cplx(M), cplx(*reversed(nm)), cplx(*reversed(nf)), cplx(*reversed(nf))
+    plan = grid_plan(3, nf, kp.nspread, kp.beta, kp.c, 1, F64, dev)
+    with plan.lock:
+        plan.setpts(xs)
+        plan.spread(c, ref)
+    stream = torch.cuda.current_stream().cuda_stream
+    before = L.nufftx_device_allocations()
+    rc = L.nufftx_spread_noalloc(3, (ctypes.c_int64 * 3)(*nf), kp.nspread, kp.beta, kp.c, F64, M, *[x.data_ptr() for x in xs],
+                                 c.data_ptr(), out.data_ptr(), ctypes.c_void_p(stream))
+    assert rc == 0, L.nufftx_last_error()
+    assert L.nufftx_device_allocations() == before
+    assert _rel(out, ref) < 1e-12
+
+    adjoint = Plan.transform(1, 3, nm, 1, 1e-12, 1, 2.0, F64, 0, dev)  # the vjp of a type 2 of sign -1
+    adjoint.setpts(xs)
+    want = torch.empty_like(f)
+    adjoint.execute(c, want)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        plan2 = Plan.transform(2, 3, nm, 1, 1e-12, -1, 2.0, F64, 0, dev)
+        plan2.setpts(xs)
+        before = L.nufftx_device_allocations()
+        got = torch.zeros_like(f)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            plan2.vjp(f, c, got, [None, None, None])
+        for _ in range(3):
+            got.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert _rel(got, want) < 1e-12
+        got.zero_()
+        plan2.vjp(f, c, got, [None, None, None])
+        torch.cuda.synchronize()
+    assert _rel(got, want) < 1e-12
+    assert L.nufftx_device_allocations() == before
