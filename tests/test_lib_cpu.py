@@ -414,3 +414,29 @@ def test_lazy_views_reach_the_library_as_values(monkeypatch):
         for want in inputs:
             assert any(t.numel() == want.numel() and t.is_complex() == want.is_complex()
                        and torch.equal(t.reshape(-1), want.reshape(-1)) for t in plan.seen)
+
+
+def _kernel_metadata():
+    """Name -> metadata of every kernel in the library (the AMDGPU notes of its code objects)."""
+    import struct
+
+    from nufftax_amd import _lib
+
+    msgpack = pytest.importorskip("msgpack")
+    data = open(_lib.LIB_PATH, "rb").read()
+    kernels, at = {}, data.find(b"AMDGPU\0\0")
+    while at >= 0:
+        namesz, descsz, kind = struct.unpack_from("<III", data, at - 12)
+        if namesz == 7 and kind == 32:  # NT_AMDGPU_METADATA
+            note = msgpack.unpackb(data[at + 8:at + 8 + descsz], raw=False)
+            kernels.update((k[".name"], k) for k in note.get("amdhsa.kernels", []))
+        at = data.find(b"AMDGPU\0\0", at + 8)
+    return kernels
+
+
+def test_fft_passes_call_no_function():
+    """The mixed-radix FFT passes are straight code: no scratch memory, which a call for an inner twiddle (a constant
+    function that the compiler could not inline) needs in every kernel."""
+    passes = {n: k for n, k in _kernel_metadata().items() if "k_fftn" in n}
+    assert len(passes) >= 30
+    assert {n for n, k in passes.items() if k[".private_segment_fixed_size"] or k.get(".uses_dynamic_stack")} == set()
