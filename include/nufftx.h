@@ -102,6 +102,12 @@ int nufftx_execute(nufftx_plan plan, void* c, void* f);
 /* Same as execute with the exponent sign overridden (type 1/2 only). */
 int nufftx_execute_sign(nufftx_plan plan, void* c, void* f, int isign);
 
+/* Device memory that a type-1/2 plan of these parameters holds, after setpts of M points, beside its fine grid, the point's
+ * sort state and records: the intermediate of the mixed-radix FFT passes and the buffers of the 3D FP64 region spread.
+ * -1 for parameters that makeplan refuses.  Makes no plan. */
+int64_t nufftx_workspace_bytes(int type, int dim, const int64_t* n_modes, int64_t n_trans, double eps, double upsampfac,
+                               int precision, int64_t M);
+
 /* nufftx_set_stream + nufftx_setpts + nufftx_execute_sign in one call (new points on every call): same arguments, checks
  * and results.  Not for plans of nufftx_plan_acquire, which keep their stream. */
 int nufftx_run(nufftx_plan plan, void* stream, int64_t M, const void* x, const void* y, const void* z, int64_t N, const void* s,

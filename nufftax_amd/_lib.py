@@ -44,6 +44,8 @@ SIGNATURES = {
     "nufftx_setpts": (ctypes.c_int, [_vp, ctypes.c_int64, _vp, _vp, _vp, ctypes.c_int64, _vp, _vp, _vp]),
     "nufftx_execute": (ctypes.c_int, [_vp, _vp, _vp]),
     "nufftx_execute_sign": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_int]),
+    "nufftx_workspace_bytes": (ctypes.c_int64, [ctypes.c_int, ctypes.c_int, _c_int64_p, ctypes.c_int64, ctypes.c_double,
+                                                ctypes.c_double, ctypes.c_int, ctypes.c_int64]),
     "nufftx_run": (ctypes.c_int, [_vp, _vp, ctypes.c_int64, _vp, _vp, _vp, ctypes.c_int64, _vp, _vp, _vp, _vp, _vp,
                                   ctypes.c_int]),
     "nufftx_execute_many": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp), ctypes.POINTER(_vp)]),
@@ -159,4 +161,12 @@ def grid_size(n_modes: int, upsampfac: float, nspread: int) -> int:
     v = lib().nufftx_grid_size(int(n_modes), float(upsampfac), int(nspread))
     if v < 0:
         raise NufftxError("nufftx_grid_size: invalid arguments")
+    return int(v)
+
+
+def workspace_bytes(kind: int, n_modes, n_trans: int, eps: float, prec: int, M: int, upsampfac: float = 2.0) -> int:
+    nm = (ctypes.c_int64 * 3)(*(list(n_modes) + [1] * (3 - len(n_modes))))
+    v = lib().nufftx_workspace_bytes(int(kind), len(n_modes), nm, int(n_trans), float(eps), float(upsampfac), int(prec), int(M))
+    if v < 0:
+        raise NufftxError("nufftx_workspace_bytes: invalid arguments")
     return int(v)

@@ -342,12 +342,6 @@ hipError_t twiddle_table(void*& dst, int n) {
   return hipSuccess;
 }
 
-int64_t fftn_mid_cells(const FftnPlan& fp, const DeconvArgs& a) {
-  const int64_t n0 = a.nm[0], f0 = a.nf[0], f1 = a.nf[1], f2 = a.nf[2];
-  if (a.dim == 1) return fp.split ? f0 : 0;
-  return a.dim == 2 ? f1 * n0 : f2 * f1 * n0;
-}
-
 template <typename T>
 struct Runner {
   const FftnPlan& fp;
@@ -529,6 +523,12 @@ bool fftn_applicable(const DeconvArgs& a) {
   return true;
 }
 
+int64_t fftn_mid_bytes(const DeconvArgs& a) {
+  const int64_t n0 = a.nm[0], f0 = a.nf[0], f1 = a.nf[1], f2 = a.nf[2];
+  const int64_t cells = a.dim == 1 ? (axis_fits(a.nf[0], a.prec) ? 0 : f0) : a.dim == 2 ? f1 * n0 : f2 * f1 * n0;
+  return cells * a.n_trans * (a.prec == kF32 ? 8 : 16);
+}
+
 hipError_t fftn_plan_init(FftnPlan& fp, const DeconvArgs& a) {
   hipError_t e;
   int len[3] = {a.nf[0], a.nf[1], a.nf[2]}, n = a.dim;
@@ -544,7 +544,7 @@ hipError_t fftn_plan_init(FftnPlan& fp, const DeconvArgs& a) {
     e = a.prec == kF32 ? twiddle_table<float>(fp.axis[d].tw, len[d]) : twiddle_table<double>(fp.axis[d].tw, len[d]);
     if (e != hipSuccess) return e;
   }
-  const int64_t bytes = fftn_mid_cells(fp, a) * a.n_trans * (a.prec == kF32 ? 8 : 16);
+  const int64_t bytes = fftn_mid_bytes(a);
   return bytes > 0 ? dev_malloc(&fp.mid, (size_t)bytes) : hipSuccess;
 }
 

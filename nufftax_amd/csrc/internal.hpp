@@ -233,6 +233,7 @@ hipError_t launch_interp_grad(const GridOpArgs& a, const void* G, const void* P,
 // ---- spread64.hip: 3D FP64 spreading by output regions
 constexpr int64_t kSpread64MinPoints = 2048;
 bool spread64_applicable(const Geometry& g, int prec, int64_t M);
+int64_t spread64_bytes(const Geometry& g, int64_t M, int64_t n_trans);  // of the buffers
 hipError_t spread64_reserve(PointSet& ps, const Geometry& g, int64_t n_trans);  // buffers for M points
 bool spread64_reserved(const PointSet& ps, const Geometry& g, int64_t n_trans);
 hipError_t launch_spread64(const GridOpArgs& a, const void* c, void* fw, hipStream_t s);  // of a reserved point set
@@ -287,6 +288,7 @@ struct FftnPlan {
   void* mid = nullptr;   // one intermediate for n_trans transforms
 };
 bool fftn_applicable(const DeconvArgs& a);
+int64_t fftn_mid_bytes(const DeconvArgs& a);  // of the intermediate
 hipError_t fftn_plan_init(FftnPlan& fp, const DeconvArgs& a);  // tables and intermediate (no allocation at run time)
 void fftn_plan_free(FftnPlan& fp);
 // spread grid -> deconvolved modes (overwrites the grid), and modes -> transformed grid

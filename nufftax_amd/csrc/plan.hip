@@ -677,6 +677,33 @@ int64_t nufftx_grid_size(int64_t n_modes, double upsampfac, int nspread) {
   return grid_size(n_modes, upsampfac, nspread);
 }
 
+int64_t nufftx_workspace_bytes(int type, int dim, const int64_t* n_modes, int64_t n_trans, double eps, double upsampfac,
+                               int precision, int64_t M) {
+  if (check_plan_args(type, dim, n_modes, n_trans, eps, upsampfac, precision, 0) || type == 3 || M < 0) return -1;
+  Geometry g;
+  double beta, kc;
+  g.dim = dim;
+  kernel_params(eps, upsampfac, g.ns, beta, kc);
+  DeconvArgs a;
+  a.dim = dim;
+  a.prec = precision;
+  a.n_trans = n_trans;
+  a.modeord = 0;
+  a.from_phihat = false;
+  for (int d = 0; d < 3; ++d) {
+    const int64_t nf = d < dim ? grid_size(n_modes[d], upsampfac, g.ns) : 1;
+    if (nf > (1LL << 30)) return -1;
+    g.nf[d] = a.nf[d] = (int)nf;
+    a.nm[d] = d < dim ? (int)n_modes[d] : 1;
+    a.fac[d] = nullptr;
+  }
+  choose_bins(g, precision, lds_budget_bytes());
+  int64_t bytes = 0;
+  if (!std::getenv("NUFFTX_ROCFFT") && !fft2_applicable(a) && fftn_applicable(a)) bytes += fftn_mid_bytes(a);
+  if (spread64_applicable(g, precision, M)) bytes += spread64_bytes(g, M, n_trans);
+  return bytes;
+}
+
 int nufftx_makeplan(int type, int dim, const int64_t* n_modes, int isign, int64_t n_trans, double eps,
                     double upsampfac, int precision, int modeord, void* stream, nufftx_plan* out) {
   if (!out) return fail(NUFFTX_ERR_INVALID_ARG, "plan output pointer is null");

@@ -531,6 +531,12 @@ bool spread64_applicable(const Geometry& g, int prec, int64_t M) {
          M * 3 * g.ns * (int64_t)sizeof(double) <= kTabMaxBytes && z.tasks <= INT32_MAX;
 }
 
+int64_t spread64_bytes(const Geometry& g, int64_t M, int64_t n_trans) {
+  const Sizes64 z = sizes64(g, M);
+  return M * (3 * g.ns * (int64_t)sizeof(double) + (int64_t)sizeof(int4)) + n_trans * M * (int64_t)(sizeof(double2) + sizeof(int2)) +
+         z.tasks * (int64_t)sizeof(int4) + (z.regions + 4) * (int64_t)sizeof(int32_t);
+}
+
 // Buffers of a spread, the largest last: a set that cannot be had leaves the small ones only.
 hipError_t spread64_reserve(PointSet& ps, const Geometry& g, int64_t n_trans) {
   const Sizes64 z = sizes64(g, ps.M);

@@ -89,12 +89,14 @@ class ServeRequest:
 
 
 def request_bytes(kind, dim, M, n_modes, eps, complex_bytes=8, n_trans=1):
-    """HBM held by one request in flight: points, strengths, output, plan fine grid and sort state."""
+    """HBM held by one request in flight: points, strengths, output, plan fine grid, sort state, and the plan's FFT
+    intermediate and FP64 spreading buffers (many times the rest for 3D complex128 points)."""
     kp = compute_kernel_params(eps)
     nf = math.prod(compute_grid_size(n, 2.0, kp.nspread) for n in n_modes)
     nm = math.prod(n_modes)
     real = complex_bytes // 2
-    return int(M * (dim * real + 4) + n_trans * (M + nm) * complex_bytes + n_trans * nf * complex_bytes)
+    extra = _lib.workspace_bytes(kind, n_modes, n_trans, eps, F64 if complex_bytes == 16 or eps < 1e-7 else F32, M)
+    return int(M * (dim * real + 4) + n_trans * (M + nm) * complex_bytes + n_trans * nf * complex_bytes) + extra
 
 
 class NufftServer:

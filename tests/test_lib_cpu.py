@@ -440,3 +440,21 @@ def test_fft_passes_call_no_function():
     passes = {n: k for n, k in _kernel_metadata().items() if "k_fftn" in n}
     assert len(passes) >= 30
     assert {n for n, k in passes.items() if k[".private_segment_fixed_size"] or k.get(".uses_dynamic_stack")} == set()
+
+
+def test_request_bytes_count_the_fp64_workspaces():
+    """The admission budget counts what an FP64 3D plan holds beside its grid: the region spread's buffers (3 ns weights, a
+    support start, and per transform a strength and a list entry per point) and half a grid for the FFT passes."""
+    from nufftax_amd import serving as S
+
+    M, n, ns = 500_000, 64, 14
+    assert R.compute_kernel_params(1e-12).nspread == ns
+    plain = M * (3 * 8 + 4) + (M + n**3) * 16 + (2 * n) ** 3 * 16
+    regions = M * (3 * ns * 8 + 16) + M * (16 + 8)
+    mid = (2 * n) ** 2 * n * 16
+    got = S.request_bytes(1, 3, M, (n, n, n), 1e-12, 16)
+    assert plain + regions + mid <= got <= 1.05 * (plain + regions + mid)
+    assert S.request_bytes(2, 3, M, (n, n, n), 1e-12, 16) == got  # its vjp spreads
+    # per transform: strengths, list, output, grid and intermediate
+    more = S.request_bytes(1, 3, M, (n, n, n), 1e-12, 16, n_trans=3) - got
+    assert more == 2 * (M * 24 + (M + n**3) * 16 + (2 * n) ** 3 * 16 + mid)
