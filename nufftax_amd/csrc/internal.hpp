@@ -232,7 +232,7 @@ hipError_t launch_interp_grad(const GridOpArgs& a, const void* G, const void* P,
 
 // ---- spread64.hip: 3D FP64 spreading by output regions
 constexpr int64_t kSpread64MinPoints = 2048;
-bool spread64_applicable(const Geometry& g, int prec, int64_t M);
+bool spread64_applicable(const Geometry& g, int prec, int64_t M, int64_t n_trans);
 int64_t spread64_bytes(const Geometry& g, int64_t M, int64_t n_trans);  // of the buffers
 hipError_t spread64_reserve(PointSet& ps, const Geometry& g, int64_t n_trans);  // buffers for M points
 bool spread64_reserved(const PointSet& ps, const Geometry& g, int64_t n_trans);

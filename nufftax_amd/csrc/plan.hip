@@ -513,7 +513,7 @@ int sort_points(nufftx_plan p, PointSet& ps, const Geometry& g, bool interp, boo
   }
   // the region spread's buffers, for type 2 too (its vjp spreads), so that no later call allocates; the atomic kernels,
   // which need none, take over where they cannot be had
-  if (&ps == &p->ps && spread64_applicable(g, p->prec, ps.M) && spread64_reserve(ps, g, p->n_trans) != hipSuccess)
+  if (&ps == &p->ps && spread64_applicable(g, p->prec, ps.M, p->n_trans) && spread64_reserve(ps, g, p->n_trans) != hipSuccess)
     (void)hipGetLastError();
   // the FP32 spreading kernels' strength bound (n_trans values and the per-block partial
   // maxima) is sized here, so that execute allocates nothing for a point set of this size
@@ -700,7 +700,7 @@ int64_t nufftx_workspace_bytes(int type, int dim, const int64_t* n_modes, int64_
   choose_bins(g, precision, lds_budget_bytes());
   int64_t bytes = 0;
   if (!std::getenv("NUFFTX_ROCFFT") && !fft2_applicable(a) && fftn_applicable(a)) bytes += fftn_mid_bytes(a);
-  if (spread64_applicable(g, precision, M)) bytes += spread64_bytes(g, M, n_trans);
+  if (spread64_applicable(g, precision, M, n_trans)) bytes += spread64_bytes(g, M, n_trans);
   return bytes;
 }
 

@@ -222,7 +222,7 @@ hipError_t spread_dim(const GridOpArgs& ga, const void* c, void* fw, hipStream_t
     return hipErrorInvalidValue;
   }
   // (clears fw itself; a point set that has no buffers for it, as nufftx_spread_noalloc's, takes the atomic kernels)
-  if (spread64_applicable(*ga.g, ga.prec, ga.ps->M) && spread64_reserved(*ga.ps, *ga.g, ga.n_trans))
+  if (spread64_applicable(*ga.g, ga.prec, ga.ps->M, ga.n_trans) && spread64_reserved(*ga.ps, *ga.g, ga.n_trans))
     return launch_spread64(ga, c, fw, s);
   if (ga.zero_out) {
     hipError_t err = launch_zero(fw, ga.n_trans * ga.g->grid_cells() * (int64_t)sizeof(cplx<T>), s);

@@ -41,8 +41,9 @@ constexpr int kWaves64 = kThreads64 / 64;
 constexpr int kCandMin = 256, kCandMax = 2048;  // candidates per task (Sizes64)
 constexpr int kRunsMax = 256;                // runs of consecutive bins around a region
 constexpr int kListMax = 128;                // points waiting for the matrix products, per wave
-// bytes of weights that a spread keeps at most; larger point sets take the atomic kernels
-constexpr int64_t kTabMaxBytes = (int64_t)2 << 30;
+// bytes of weights and of all buffers that a spread keeps at most; more points or transforms take the atomic kernels
+// (24 bytes per point and transform: the bound also keeps the counter of pairs in 31 bits)
+constexpr int64_t kTabMaxBytes = (int64_t)2 << 30, kMaxBytes64 = (int64_t)4 << 30;
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
@@ -521,14 +522,15 @@ int64_t runs64(const Geometry& g) {  // most runs around a region
 // and 10 from 100 regions on (50k points, ns = 8: 48^3 grid, 54 regions, 133 -> 172 us, 128^3, 1024 regions, 439 ->
 // 259 us; 30k points, ns = 10: 40^3, 45 regions, 132 -> 168 us, 64^3, 128 regions, 296 -> 183 us); not below (50k
 // points on 128^3: ns = 6 299 -> 249 us uniform but 194 -> 228 us clustered, and 1M points 457 -> 826 us).
-bool spread64_applicable(const Geometry& g, int prec, int64_t M) {
+bool spread64_applicable(const Geometry& g, int prec, int64_t M, int64_t n_trans) {
   if (g.dim != 3 || prec != kF64 || g.ns < 8 || M < kSpread64MinPoints) return false;
   for (int d = 0; d < 3; ++d)
     if (g.nf[d] < g.ns) return false;
   const Sizes64 z = sizes64(g, M);
   if (g.ns < 12 && z.regions < 100) return false;
   return z.regions < INT32_MAX && runs64(g) <= kRunsMax &&
-         M * 3 * g.ns * (int64_t)sizeof(double) <= kTabMaxBytes && z.tasks <= INT32_MAX;
+         M * 3 * g.ns * (int64_t)sizeof(double) <= kTabMaxBytes && spread64_bytes(g, M, n_trans) <= kMaxBytes64 &&
+         z.tasks <= (INT32_MAX - kBlocks64) / n_trans;  // a task number per transform, and one past the last per block
 }
 
 int64_t spread64_bytes(const Geometry& g, int64_t M, int64_t n_trans) {

@@ -458,3 +458,17 @@ def test_request_bytes_count_the_fp64_workspaces():
     # per transform: strengths, list, output, grid and intermediate
     more = S.request_bytes(1, 3, M, (n, n, n), 1e-12, 16, n_trans=3) - got
     assert more == 2 * (M * 24 + (M + n**3) * 16 + (2 * n) ** 3 * 16 + mid)
+
+
+def test_fp64_region_spread_is_bounded_in_points_and_transforms():
+    """The region spread's buffers stay within 4 GiB (2 GiB of weights) whatever the number of transforms: beyond, a plan holds
+    none and takes the atomic kernels.  Its counters (pairs, tasks) are 32-bit, at 24 bytes a pair."""
+    from nufftax_amd import _lib
+    from nufftax_amd._plan import F64
+
+    held = lambda M, n_trans: _lib.workspace_bytes(1, (16, 16, 16), n_trans, 1e-12, F64, M)  # noqa: E731  (32^3: no FFT passes)
+    ns, M = 14, 2_000_000
+    for n_trans in (1, 8, 64, 70):
+        assert M * (24 * ns + 16 + 24 * n_trans) <= held(M, n_trans) <= 4 << 30
+    for M, n_trans in ((2_000_000, 75), (2_000_000, 1000), (6_300_000, 342), (6_500_000, 1), (2**31 - 2, 1), (2**31 - 2, 65535)):
+        assert held(M, n_trans) == 0
