@@ -4,8 +4,8 @@
 //   v_j = sum_z wz_j(z) sum_y wy_j(y) sum_x F[z][y][x] wx_j(x)        (nufftax/core/spread.py:661-715)
 // so for 16 points the x sums of one z slice and part are one matrix product G = F Bx.  F and wx are split into
 // two fp16 parts (hi + lo: 22 bits and more, scaled to the top of fp16's range, as in the spread), and the K = 32 of
-// v_mfma_f32_16x16x32_f16 holds the 16 x twice, [F_hi | F_lo] against [B_hi ; B_hi] and then [B_lo ; B_lo]: all four
-// products in two instructions, nothing left out but the roundings of lo.  The tile is staged in LDS already split,
+// v_mfma_f32_16x16x32_f16 holds the 16 x twice, [F_lo | F_hi] against [B_lo ; B_lo] and then [B_hi ; B_hi]: all four
+// products in two instructions, nothing left out but the roundings of lo, the small ones summed first.  The tile is staged in LDS already split,
 // as four fp16 planes (re and im, hi and lo: 8 bytes a cell, as FP32), so that a lane reads 8 cells of one plane
 // with one 16-byte read, its operand; a window is read once per sub-bin that a wave visits, into (4 + ns) * 8
 // registers.  A group then costs two MFMAs and 5 FMAs per slice and part.  (Windows read from the grid by each wave,
@@ -22,7 +22,8 @@
 //   2. contiguous ranges of groups per wave; per group the lanes evaluate the 3 ns weights of the 16 points into LDS
 //      rows with zeros around them (read at the point's offset in the window), then multiply.
 // A tile that holds a non-finite value would spread it through the zero weights: its points take their own cells
-// one by one.
+// one by one.  So do points whose result is small beside the tile's largest value (2^-13), whose cells the common
+// scale of the tile leaves too few bits.
 //
 // MFMA operand layout: A[i][k] in lane i + 16 (k / 8), element k % 8; B[k][j] in lane j + 16 (k / 8), element k % 8;
 // D[i][j] in lane j + 16 (i / 4), element i % 4.
@@ -59,13 +60,35 @@ __host__ __device__ inline Gather3Tile gather3_tile(const int (&bs)[3], int ns) 
 constexpr int kG3Quads = 6;  // four-cell pieces of the tile per thread: 24 x 16 x 16 cells
 
 struct Gather3Lds {
-  uint3 word[kG3MaxSub];       // tile-relative words of the points (compact_word's layout)
+  uint3 word[kG3MaxSub];       // tile-relative words of the points (g3_word)
   uint16_t order[kG3Order];
   alignas(16) float wave[kG3Waves][kG3WaveF];
   unsigned short wcnt[kG3Ppt * kG3Waves * 16];
   int cnt[16], start[17];
   unsigned smax;
 };
+
+// tile-relative word of one coordinate: support start - org << 25 | round((t + ns/2) 2^25), t = start - xs.  (The compact
+// records' 2^-24 cells would be the next largest error of the gather after the FP32 sums.)
+template <int NS>
+__device__ __forceinline__ unsigned g3_word(double x, int nf, int org) {
+  const Folded f = fold_coord(x, nf);
+  const int i0 = support_start(f, NS / 2);
+  const double u = ((double)i0 - f.xs + (double)(NS / 2)) * 33554432.0;  // 2^25
+  return ((unsigned)(i0 - org) << 25) | (unsigned)fmin(fmax(rint(u), 0.0), 33554431.0);
+}
+
+// Results below this (in the products' units, where the tile's largest value is about 2^29) are taken from the cells instead:
+// an fp16 lo part resolves 2^-24 at least (the matrix cores take subnormal fp16 operands as they are), so the products of a
+// cell are off by up to 2^-11 of these units, which a sum of 2^16 carries in its last FP32 bits.
+constexpr float kG3Small = 65536.0f;
+
+// sum over the four lanes i, i + 16, i + 32, i + 48 of a point
+template <typename T>
+__device__ __forceinline__ T quad_sum(T v) {
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
 
 template <typename CT, int NS, bool POLY>
 __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, const cplx<float>* __restrict__ fw,
@@ -123,9 +146,9 @@ __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, 
         const int p = a.perm[sd.y + base + j];
         uint3 w = make_uint3(0u, 0u, 0u);
         if ((unsigned)p < (unsigned)a.M) {
-          w.x = pack_compact<NS>((double)static_cast<const CT*>(a.coord[0])[p], a.nf[0], org[0]);
-          w.y = pack_compact<NS>((double)static_cast<const CT*>(a.coord[1])[p], a.nf[1], org[1]);
-          w.z = pack_compact<NS>((double)static_cast<const CT*>(a.coord[2])[p], a.nf[2], org[2]);
+          w.x = g3_word<NS>((double)static_cast<const CT*>(a.coord[0])[p], a.nf[0], org[0]);
+          w.y = g3_word<NS>((double)static_cast<const CT*>(a.coord[1])[p], a.nf[1], org[1]);
+          w.z = g3_word<NS>((double)static_cast<const CT*>(a.coord[2])[p], a.nf[2], org[2]);
         }
         L.word[j] = w;
         const int sx = min((int)(w.x >> 25) / kW3SB, nsx - 1), sy = min((int)(w.y >> 25) / kW3SB, nsy - 1);
@@ -239,9 +262,9 @@ __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, 
           ++s;
         } while (s < 15 && L.start[s + 1] <= kG3K * g);
         next = L.start[s + 1];
-        // the window: lane (y = i, kq) takes x = 8 (kq & 1) .. + 7 of row i of every slice, of the hi (kq < 2) or lo plane
+        // the window: lane (y = i, kq) takes x = 8 (kq & 1) .. + 7 of row i of every slice, of the lo (kq < 2) or hi plane
         const int at = ((s / (nsx * nsy) * kW3SBZ) * T.ty + (s / nsx % nsy) * kW3SB + i) * T.tx + (s % nsx) * kW3SB + 8 * (kq & 1) +
-                       (kq >> 1) * T.cells;
+                       (kq < 2 ? T.cells : 0);
 #pragma unroll
         for (int z = 0; z < WZ; ++z) {
           fre[z] = *reinterpret_cast<const wh_h8*>(planes + at + z * T.ty * T.tx);
@@ -256,10 +279,10 @@ __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, 
           const unsigned wd = real ? word[3 * slot + kq] : 0u;
           float wt[NS];
           if constexpr (POLY) {
-            // v = 2 (t + NS/2) - 1 = (u - 3 2^23) 2^-23 exactly (|u - 3 2^23| <= 2^23); padding (u = 0) takes v = -1
-            es_poly_weights<NS>(fmaxf((float)((int)(wd & 0x1FFFFFFu) - 3 * 8388608) * (1.0f / 8388608.0f), -1.0f), a.poly, wt);
+            // v = 2 (t + NS/2) - 1, exactly (|u - 2^24| <= 2^24)
+            es_poly_weights<NS>((float)((int)(wd & 0x1FFFFFFu) - 16777216) * (1.0f / 16777216.0f), a.poly, wt);
           } else {
-            const float t = (float)((double)(wd & 0x1FFFFFFu) * (1.0 / 16777216.0) - (double)(NS / 2 + 1));
+            const float t = (float)((double)(wd & 0x1FFFFFFu) * (1.0 / 33554432.0) - (double)(NS / 2));
 #pragma unroll
             for (int m = 0; m < NS; ++m) wt[m] = es_phi_in(t + (float)m, a.es.beta_log2e, a.es.c);
           }
@@ -275,6 +298,7 @@ __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, 
       wave_sync_win();
       const int4 mt = meta[i];
       float sr = 0.0f, si = 0.0f;
+      bool cells = !fine;
       if (fine) {
         float bx[8], wy[4];
 #pragma unroll
@@ -284,6 +308,10 @@ __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, 
         wh_h8 bh, bl;
         split_f16(bx, bh, bl);
         const win_f4 zero4 = {0.f, 0.f, 0.f, 0.f};
+        // The sums over slices and lanes in FP64 make up for the split's roundings: relative l2 1.12e-7 on random grids, the
+        // gather of one thread per point 1.16e-7 (two or six slices summed in FP32 first: 1.17 and 1.20e-7; 8M clustered
+        // points, 128^3 modes, whole type 2 1365 us, with those 1342 and 1322).
+        double zr = 0.0, zi = 0.0;
 #pragma unroll
         for (int z = 0; z < WZ; ++z) {
           win_f4 gr = __builtin_amdgcn_mfma_f32_16x16x32_f16(fre[z], bl, zero4, 0, 0, 0);
@@ -297,32 +325,50 @@ __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, 
             pr = fmaf(gr[e], wy[e], pr);
             pi = fmaf(gi[e], wy[e], pi);
           }
-          sr = fmaf(pr, wz, sr);
-          si = fmaf(pi, wz, si);
+          zr = fma((double)pr, (double)wz, zr);
+          zi = fma((double)pi, (double)wz, zi);
         }
+        sr = (float)quad_sum(zr + (double)sr);
+        si = (float)quad_sum(zi + (double)si);
+        cells = fm > 0.0f && fmaxf(fabsf(sr), fabsf(si)) < kG3Small;
         sr = ldexpf(sr, kout);
         si = ldexpf(si, kout);
-      } else if (mt.w >= 0) {
-        // support rows of the point, lane kq the slices kq, kq + 4, ..: its own cells only
-        const int slot = L.order[kG3K * g + i];
-        const uint3 w = L.word[slot];
-        const int x0 = org[0] + (int)(w.x >> 25), y0 = org[1] + (int)(w.y >> 25), z0 = org[2] + (int)(w.z >> 25);
-        for (int z = kq; z < NS; z += 4)
-          for (int y = 0; y < NS; ++y) {
-            const float wzy = rowz[kW3RowZ * i + kW3SBZ + z] * rowy[kWinRow * i + (16 - NS) + y];
-            const cplx<float>* src = fT + ((int64_t)wrap_idx(z0 + z, a.nf[2]) * a.nf[1] + wrap_idx(y0 + y, a.nf[1])) * a.nf[0];
-            for (int x = 0; x < NS; ++x) {
-              const cplx<float> v = src[wrap_idx(x0 + x, a.nf[0])];
-              const float wt = wzy * (rowx[kWinRow * i + (16 - NS) + x] * (1.0f / 16384.0f));
-              sr = fmaf(v.re, wt, sr);
-              si = fmaf(v.im, wt, si);
-            }
-          }
       }
-      sr += __shfl_xor(sr, 16, 64);
-      si += __shfl_xor(si, 16, 64);
-      sr += __shfl_xor(sr, 32, 64);
-      si += __shfl_xor(si, 32, 64);
+      cells = cells && mt.w >= 0;
+      if (__any(cells)) {  // (rare, or a tile that is not finite)
+        // support rows of the point, lane kq the slices kq, kq + 4, ..: its own cells only, in FP32
+        float cr = 0.0f, ci = 0.0f;
+        if (cells) {
+          const int slot = L.order[kG3K * g + i];
+          const uint3 w = L.word[slot];
+          const int x0 = org[0] + (int)(w.x >> 25), y0 = org[1] + (int)(w.y >> 25), z0 = org[2] + (int)(w.z >> 25);
+          for (int z = kq; z < NS; z += 4) {
+            float pr = 0.0f, pi = 0.0f;
+            for (int y = 0; y < NS; ++y) {
+              const cplx<float>* src = fT + ((int64_t)wrap_idx(z0 + z, a.nf[2]) * a.nf[1] + wrap_idx(y0 + y, a.nf[1])) * a.nf[0];
+              float rr = 0.0f, ri = 0.0f;
+              for (int x = 0; x < NS; ++x) {
+                const cplx<float> v = src[wrap_idx(x0 + x, a.nf[0])];
+                const float wx = rowx[kWinRow * i + (16 - NS) + x] * (1.0f / 16384.0f);
+                rr = fmaf(v.re, wx, rr);
+                ri = fmaf(v.im, wx, ri);
+              }
+              const float wy = rowy[kWinRow * i + (16 - NS) + y];
+              pr = fmaf(rr, wy, pr);
+              pi = fmaf(ri, wy, pi);
+            }
+            const float wz = rowz[kW3RowZ * i + kW3SBZ + z];
+            cr = fmaf(pr, wz, cr);
+            ci = fmaf(pi, wz, ci);
+          }
+        }
+        cr = quad_sum(cr);
+        ci = quad_sum(ci);
+        if (cells) {
+          sr = cr;
+          si = ci;
+        }
+      }
       if (kq == 0 && (unsigned)mt.w < (unsigned)a.M) out[(int64_t)tr * a.M + mt.w] = cplx<float>{sr, si};
       wave_sync_win();  // the next group overwrites the rows
     }
