@@ -94,7 +94,8 @@ template <typename CT, int NS, bool POLY>
 __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, const cplx<float>* __restrict__ fw,
                                                                cplx<float>* __restrict__ out) {
   constexpr int WZ = kW3SBZ + NS;
-  constexpr uint16_t kPad = 0xFFFF;
+  constexpr uint16_t kPad = 0xFFFF, kBad = 0x8000;  // entries of the order: slot, and a mark
+  static_assert(kG3MaxSub < kBad, "slots leave the mark free");
   __shared__ __align__(16) Gather3Lds L;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   _Float16* const planes = reinterpret_cast<_Float16*>(smem_raw);  // [re hi, re lo, im hi, im lo][z][y][x]
@@ -138,19 +139,24 @@ __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, 
     if (tid < kG3Ppt * kG3Waves * 16 / 2) reinterpret_cast<unsigned*>(L.wcnt)[tid] = 0u;
     __syncthreads();
     int sb[kG3Ppt], rank[kG3Ppt];
+    bool bad[kG3Ppt];  // a coordinate is not finite: NaN weights, a NaN result
 #pragma unroll
     for (int r = 0; r < kG3Ppt; ++r) {
       const int j = tid + r * kG3Threads;
       sb[r] = -1;
+      bad[r] = false;
       if (base + j < sd.z) {
         const int p = a.perm[sd.y + base + j];
         uint3 w = make_uint3(0u, 0u, 0u);
+        double xyz[3] = {0.0, 0.0, 0.0};
         if ((unsigned)p < (unsigned)a.M) {
-          w.x = g3_word<NS>((double)static_cast<const CT*>(a.coord[0])[p], a.nf[0], org[0]);
-          w.y = g3_word<NS>((double)static_cast<const CT*>(a.coord[1])[p], a.nf[1], org[1]);
-          w.z = g3_word<NS>((double)static_cast<const CT*>(a.coord[2])[p], a.nf[2], org[2]);
+#pragma unroll
+          for (int d = 0; d < 3; ++d) xyz[d] = (double)static_cast<const CT*>(a.coord[d])[p];
+          w = make_uint3(g3_word<NS>(xyz[0], a.nf[0], org[0]), g3_word<NS>(xyz[1], a.nf[1], org[1]),
+                         g3_word<NS>(xyz[2], a.nf[2], org[2]));
         }
         L.word[j] = w;
+        bad[r] = !(isfinite(xyz[0]) && isfinite(xyz[1]) && isfinite(xyz[2]));
         const int sx = min((int)(w.x >> 25) / kW3SB, nsx - 1), sy = min((int)(w.y >> 25) / kW3SB, nsy - 1);
         const int sz = min((int)(w.z >> 25) / kW3SBZ, nsz - 1);
         sb[r] = (sz * nsy + sy) * nsx + sx;
@@ -194,7 +200,9 @@ __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, 
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kG3Ppt; ++r)
-      if (sb[r] >= 0) L.order[L.wcnt[(r * kG3Waves + wave) * 16 + sb[r]] + rank[r]] = (uint16_t)(tid + r * kG3Threads);
+      if (sb[r] >= 0)
+        L.order[L.wcnt[(r * kG3Waves + wave) * 16 + sb[r]] + rank[r]] =
+            (uint16_t)((tid + r * kG3Threads) | (bad[r] ? kBad : 0));
     if (tid < 16 * (kG3K - 1)) {
       const int s = tid / (kG3K - 1), slot = L.start[s] + L.cnt[s] + tid % (kG3K - 1);
       if (slot < L.start[s + 1]) L.order[slot] = kPad;
@@ -273,8 +281,8 @@ __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, 
       }
       // -- weights and read indices: lanes 0-15 x, 16-31 y, 32-47 z of point i, 48-63 its index
       {
-        const int slot = L.order[kG3K * g + i];
-        const bool real = slot != kPad;
+        const int entry = L.order[kG3K * g + i], slot = entry & (kBad - 1);
+        const bool real = entry != kPad;
         if (kq < 3) {
           const unsigned wd = real ? word[3 * slot + kq] : 0u;
           float wt[NS];
@@ -286,7 +294,7 @@ __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, 
 #pragma unroll
             for (int m = 0; m < NS; ++m) wt[m] = es_phi_in(t + (float)m, a.es.beta_log2e, a.es.c);
           }
-          const float sc = kq == 0 ? 16384.0f : 1.0f;
+          const float sc = real && (entry & kBad) ? NAN : kq == 0 ? 16384.0f : 1.0f;
 #pragma unroll
           for (int m = 0; m < NS; ++m) myrow[m] = wt[m] * sc;
           const int l = (int)(wd >> 25);
@@ -339,8 +347,7 @@ __global__ void __launch_bounds__(kG3Threads, 2) k_gather_win3(SIArgs<float> a, 
         // support rows of the point, lane kq the slices kq, kq + 4, ..: its own cells only, in FP32
         float cr = 0.0f, ci = 0.0f;
         if (cells) {
-          const int slot = L.order[kG3K * g + i];
-          const uint3 w = L.word[slot];
+          const uint3 w = L.word[L.order[kG3K * g + i] & (kBad - 1)];
           const int x0 = org[0] + (int)(w.x >> 25), y0 = org[1] + (int)(w.y >> 25), z0 = org[2] + (int)(w.z >> 25);
           for (int z = kq; z < NS; z += 4) {
             float pr = 0.0f, pi = 0.0f;

@@ -1160,6 +1160,26 @@ def test_gather3_keeps_small_cells_beside_large_ones(rng, peak):
     assert R.rel_l2(out[0][far], R.interp(xs, fw[0].astype(np.complex128), kp)[far]) < 2e-6
 
 
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+def test_gather3_non_finite_coordinate_gives_nan(rng, bad, monkeypatch):
+    """A point with a non-finite coordinate, in any dimension and with either form of the kernel weights, has a NaN result; the
+    others are those without it."""
+    nfs, M = (32, 40, 36), 500
+    coords = [rng.uniform(-np.pi, np.pi, M).astype(np.float32) for _ in nfs]
+    shape = (1,) + tuple(reversed(nfs))
+    fw = (rng.standard_normal(shape) + 1j * rng.standard_normal(shape)).astype(np.complex64)
+    for poly in ("1", "0"):
+        monkeypatch.setenv("NUFFTX_ES_POLY", poly)
+        good, _, _ = _gather3(nfs, coords, fw)
+        hit = [v.copy() for v in coords]
+        for d in range(3):
+            hit[d][[7 + d, 300 + d]] = bad
+        out, _, _ = _gather3(nfs, hit, fw)
+        touched = np.isin(np.arange(M), [7, 8, 9, 300, 301, 302])
+        assert np.isnan(out[0][touched].real).all() and np.isnan(out[0][touched].imag).all()
+        assert R.rel_l2(out[0][~touched], good[0][~touched]) < 1e-6
+
+
 # ------------------------------------------------------------------ 1D without a sort
 
 
