@@ -102,9 +102,8 @@ constexpr int kWinMaxSub = 4096;
 // (its windows cost the same at every ns, and the bank-spread kernel's ns^3 atomics per point
 // are cheaper below 8: 1.06 against 1.48 ms for 8M clustered points at ns = 6), bins of whole
 // 8 x 8 x 4 sub-bins (at most 16 of them), tiles of at most 127 cells a side, subproblems of
-// at most 2048 points (four per thread of a 512-thread block)
+// at most 4096 points (eight per thread of a 512-thread block)
 constexpr int kWin3MaxSub = 4096;
-inline int win3_maxsub(int64_t M) { return M >= 256 * (kWin3MaxSub / 2) ? kWin3MaxSub : kWin3MaxSub / 2; }
 inline bool win3d_geometry(const Geometry& g, int prec, int maxsub) {
   if (g.dim != 3 || prec != 0 || g.ns != 8 || maxsub > kWin3MaxSub) return false;
   if (g.bs[0] % 8 || g.bs[1] % 8 || g.bs[2] % 4) return false;
@@ -191,6 +190,9 @@ hipError_t grow_buffer(T*& p, int64_t& cap, int64_t need, std::vector<void*>& re
   cap = n;
   return hipSuccess;
 }
+
+// points per subproblem of a set of M points that the 3D window spread takes (spread.hip)
+int win3_maxsub(const Geometry& g, int64_t M);
 
 // ---- prep.hip: sub-bin order and point records for the 2D FP32 matrix-core kernels
 bool subsort_applicable(const SortTuning& tune, const Geometry& g, int prec);

@@ -488,11 +488,8 @@ int sort_points(nufftx_plan p, PointSet& ps, const Geometry& g, bool interp, boo
   if (((spread && win_spread_enabled()) || (interp && win_interp_enabled())) && win2d_geometry(g, p->prec, kWinMaxSub) &&
       !std::getenv("NUFFTX_MAXSUB"))
     tune.maxsub = kWinMaxSub;
-  // The 3D window spread takes subproblems of up to 4096 points, one tile flush for twice the points, where subproblems of
-  // 2048 would still be one for each of the 256 CUs (8M clustered points, 64^3 modes: 1373 -> 1165 us); fewer points need
-  // the parallelism (100k clustered points, 32^3 modes: 102 us with 2048, 122 with 4096).
   if (spread && win_spread_enabled() && win3d_geometry(g, p->prec, kWin3MaxSub) && !std::getenv("NUFFTX_MAXSUB"))
-    tune.maxsub = win3_maxsub(ps.M);
+    tune.maxsub = win3_maxsub(g, ps.M);
   const bool subsort = subsort_applicable(tune, g, p->prec);
   // records pay for their cost in the sort only where the point set is interpolated;
   // the matrix-core kernels need the full records with sub-bins

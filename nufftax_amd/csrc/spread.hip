@@ -169,21 +169,23 @@ bool spread_win(const GridOpArgs& ga, const void* c, void* fw, hipStream_t s, hi
   return false;
 }
 
+// Whether the 3D window spread of subproblems of up to maxsub points has exact tiles (two 64-bit words per cell: the
+// bank-spread kernel's accuracy), the default; its static LDS (ordering counters) is below 2304 bytes.  Packed tiles
+// (one word per cell, about 3x the rounding error, 2% faster on 8M clustered points) are taken with
+// NUFFTX_WIN3_PACKED=1 or where the exact tile does not fit the LDS (grids of more than 16384 bins of 16 x 8 x 8 cells).
+bool win3_exact(const Geometry& g, int maxsub) {
+  const char* pe = std::getenv("NUFFTX_WIN3_PACKED");
+  return w3_spread_lds<false>(g.tile_cells, maxsub) + 2304 <= (size_t)lds_device_max_bytes() && !(pe && pe[0] == '1');
+}
+
 // The 3D matrix-core window spread (3D FP32, ns = 8, bins of whole 8 x 8 x 4 sub-bins,
-// subproblems of <= 2048 points): points packed in sorted order, then spread.  Exact tiles
-// (two 64-bit words per cell: the bank-spread kernel's accuracy) are the default; packed
-// tiles (one word per cell, about 3x the rounding error, 2% faster on 8M clustered points)
-// are taken with NUFFTX_WIN3_PACKED=1 or where the exact tile does not fit the LDS.
+// subproblems of <= 4096 points): points packed in sorted order, then spread.
 bool spread_win3d(const GridOpArgs& ga, const void* c, void* fw, hipStream_t s, hipError_t& err) {
   PointSet& ps = const_cast<PointSet&>(*ga.ps);
   if (!win3d_geometry(*ga.g, ga.prec, ps.maxsub) || !ps.has_slot || !win_spread_enabled()) return false;
   SIArgs<float> a = make_si_args<float>(ga);
-  // the static LDS (ordering counters) is below 2304 bytes
-  const size_t lds_exact = w3_spread_lds<false>(ga.g->tile_cells, ps.maxsub);
-  const size_t lds_packed = w3_spread_lds<true>(ga.g->tile_cells, ps.maxsub);
-  const char* pe = std::getenv("NUFFTX_WIN3_PACKED");
-  const bool exact = lds_exact + 2304 <= (size_t)lds_device_max_bytes() && !(pe && pe[0] == '1');
-  const size_t lds = exact ? lds_exact : lds_packed;
+  const bool exact = win3_exact(*ga.g, ps.maxsub);
+  const size_t lds = exact ? w3_spread_lds<false>(ga.g->tile_cells, ps.maxsub) : w3_spread_lds<true>(ga.g->tile_cells, ps.maxsub);
   if (lds + 2304 > (size_t)lds_device_max_bytes()) return false;
   const int64_t grid_bytes = ga.n_trans * ga.g->grid_cells() * (int64_t)sizeof(cplx<float>);
   const bool fused_zero = ga.zero_out && grid_bytes % 16 == 0;
@@ -288,6 +290,14 @@ hipError_t spread_many_impl(const GridOpArgs* gas, int count, const void* const*
 }
 
 }  // namespace
+
+// Subproblems of 4096 points, one tile flush for twice the points, where subproblems of 2048 would still be one for each of
+// the 256 CUs (8M clustered points, 64^3 modes: 1373 -> 1165 us; fewer points need the parallelism: 100k clustered points,
+// 32^3 modes, 102 us with 2048, 122 with 4096) and the tile is exact: a packed tile's resolution is that of the sum of the
+// subproblem's strengths, and twice the points would cost a bit.
+int win3_maxsub(const Geometry& g, int64_t M) {
+  return M >= 256 * (kWin3MaxSub / 2) && win3_exact(g, kWin3MaxSub) ? kWin3MaxSub : kWin3MaxSub / 2;
+}
 
 hipError_t launch_spread_many(const GridOpArgs* gas, int count, const void* const* c, void* const* fw, hipStream_t s) {
   if (count < 1 || count > kMaxMany) return hipErrorNotSupported;

@@ -1180,6 +1180,37 @@ def test_gather3_non_finite_coordinate_gives_nan(rng, bad, monkeypatch):
         assert R.rel_l2(out[0][~touched], good[0][~touched]) < 1e-6
 
 
+def test_spread3d_packed_tiles_keep_their_subproblems(monkeypatch):
+    """Grids of more than 16384 bins spread into packed tiles, whose resolution falls with the points of a subproblem: 600k
+    points in some 60 of its bins are as far from the FP64 spread as with subproblems of 2048 points."""
+    from nufftax_amd._plan import F32, F64, Plan
+
+    rng = np.random.default_rng(5)
+    nfs, M, dev = (288, 288, 256), 600_000, torch.device(DEV, 0)
+    assert (nfs[0] // 16) * (nfs[1] // 8) * (nfs[2] // 8) > 16384
+    kp = R.compute_kernel_params(1e-7)
+    coords = [rng.uniform(0.0, 1.1, M).astype(np.float32) for _ in nfs]
+    c = (rng.standard_normal(M) + 1j * rng.standard_normal(M)).astype(np.complex64)
+
+    def spread(prec, rdt, cdt):
+        plan = Plan.grid_op(3, nfs, kp.nspread, kp.beta, kp.c, 1, prec, dev)
+        plan.setpts([_t(x, rdt) for x in coords])
+        fw = torch.empty(tuple(reversed(nfs)), dtype=cdt, device=DEV)
+        plan.spread(_t(c, cdt), fw)
+        return fw.to(torch.complex128)
+
+    want = spread(F64, torch.float64, torch.complex128)
+    err = []
+    for maxsub in ("2048", None):
+        if maxsub:
+            monkeypatch.setenv("NUFFTX_MAXSUB", maxsub)
+        else:
+            monkeypatch.delenv("NUFFTX_MAXSUB")
+        err.append(float(torch.linalg.vector_norm(spread(F32, torch.float32, torch.complex64) - want)
+                         / torch.linalg.vector_norm(want)))
+    assert err[1] < 1.1 * err[0], err
+
+
 # ------------------------------------------------------------------ 1D without a sort
 
 
