@@ -44,7 +44,7 @@
 namespace nufftx {
 
 constexpr int kW3Threads = 512;                    // 8 waves per subproblem
-constexpr int kW3Ppt = 8;                          // points per thread while ordering
+constexpr int kW3Ppt = 8;                          // points per thread while ordering, at most
 constexpr int kW3K = 32;                           // points per group
 constexpr int kW3Hold = 10;                        // groups summed in FP32 before they go to the exact tile
 constexpr int kW3SB = 8;                           // sub-bin side in x and y (support starts)
@@ -70,7 +70,8 @@ inline size_t w3_spread_lds(int64_t tile_cells, int maxsub) {
          (size_t)(kW3Threads / 64) * kW3WaveF * sizeof(float);
 }
 
-template <int NS, bool PK>
+// PPT: points per thread while ordering (4 or 8; subproblems of up to 512 PPT points)
+template <int NS, bool PK, int PPT>
 __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, int maxsub,
                                                               const uint4* __restrict__ words,
                                                               const float2* __restrict__ cs,
@@ -87,7 +88,7 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
   Word* tile = reinterpret_cast<Word*>(smem_raw);  // packed words, or real parts
   Word* tim = tile + TC;                            // imaginary parts (exact tiles)
   uint16_t* order = reinterpret_cast<uint16_t*>(tile + (PK ? 1 : 2) * TC);
-  __shared__ unsigned short wcnt[kW3Ppt * W * 16];
+  __shared__ unsigned short wcnt[PPT * W * 16];
   __shared__ int cnt[16], start[17];
   __shared__ unsigned smax;
   __shared__ float ssum[W];
@@ -117,7 +118,7 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
     }
   for (int e = lane; e < kW3RowZF; e += 64)
     if (e % kW3RowZ < kW3SBZ || e % kW3RowZ >= kW3SBZ + NS || e >= kW3K * kW3RowZ) rowz[e] = 0.0f;
-  for (int e = tid; e < kW3Ppt * W * 16; e += kW3Threads) wcnt[e] = 0;
+  for (int e = tid; e < PPT * W * 16; e += kW3Threads) wcnt[e] = 0;
   if (tid == 0) smax = 0u;
   __syncthreads();
 
@@ -127,12 +128,12 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
     const int sz = min((int)(p.z >> 25) / kW3SBZ, nsz - 1);
     return (sz * nsy + sy) * nsx + sx;
   };
-  int sb[kW3Ppt];
+  int sb[PPT];
   unsigned mymax = 0;
   float mysum = 0.0f;
   const int npass = (n + kW3Threads - 1) / kW3Threads;
 #pragma unroll
-  for (int r = 0; r < kW3Ppt; ++r) {
+  for (int r = 0; r < PPT; ++r) {
     const int j = tid + r * kW3Threads;
     sb[r] = -1;
     if (j < n) {
@@ -143,9 +144,9 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
       mysum += fmaxf(are, aim) + 0.0f * (are + aim);  // NaN in either part propagates
     }
   }
-  int rank[kW3Ppt];
+  int rank[PPT];
 #pragma unroll
-  for (int r = 0; r < kW3Ppt; ++r) {
+  for (int r = 0; r < PPT; ++r) {
     if (r >= npass) break;
     const bool valid = sb[r] >= 0;
     uint64_t m = __ballot(valid);
@@ -168,9 +169,9 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
   }
   __syncthreads();
   if (tid < 16) {  // counts per sub-bin, padded starts (16 lanes of one wave), first slot of every (pass, wave) run
-    int v[kW3Ppt * W], c = 0;
+    int v[PPT * W], c = 0;
 #pragma unroll
-    for (int e = 0; e < kW3Ppt * W; ++e) {
+    for (int e = 0; e < PPT * W; ++e) {
       v[e] = wcnt[e * 16 + tid];
       c += v[e];
     }
@@ -186,14 +187,14 @@ __global__ void __launch_bounds__(kW3Threads) k_spread_win3dh(SIArgs<float> a, i
     if (tid == 15) start[16] = incl;
     int run = incl - padded;
 #pragma unroll
-    for (int e = 0; e < kW3Ppt * W; ++e) {
+    for (int e = 0; e < PPT * W; ++e) {
       wcnt[e * 16 + tid] = (unsigned short)run;
       run += v[e];
     }
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < kW3Ppt; ++r)
+  for (int r = 0; r < PPT; ++r)
     if (r < npass && sb[r] >= 0) order[wcnt[(r * W + wave) * 16 + sb[r]] + rank[r]] = (uint16_t)(tid + r * kW3Threads);
   if (tid < 16 * (kW3K - 1)) {
     const int s = tid / (kW3K - 1), q = tid % (kW3K - 1);

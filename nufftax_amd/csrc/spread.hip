@@ -195,7 +195,11 @@ bool spread_win3d(const GridOpArgs& ga, const void* c, void* fw, hipStream_t s, 
     return true;
   // ns = 8 (win3d_geometry); the exp form of the kernel weights (the polynomial form spilled
   // scalar registers here and was 0.035 ms slower on 8M clustered points)
-  auto kern = exact ? k_spread_win3dh<8, false> : k_spread_win3dh<8, true>;
+  // subproblems of 2048 points are ordered with four points per thread, half the passes and counters of eight (a type 1 of
+  // 2000 points, 16^3 modes: 59.0 us with eight, 51.7 with four; 100k points, 45^3: 172 and 164)
+  const bool half = ps.maxsub <= kWin3MaxSub / 2;
+  auto kern = half ? (exact ? k_spread_win3dh<8, false, kW3Ppt / 2> : k_spread_win3dh<8, true, kW3Ppt / 2>)
+                   : (exact ? k_spread_win3dh<8, false, kW3Ppt> : k_spread_win3dh<8, true, kW3Ppt>);
   if (lds > 65536) (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   hipLaunchKernelGGL(kern, dim3(ps.max_subprob, (unsigned)ga.n_trans), dim3(kW3Threads), lds, s, a, ps.maxsub,
                      ps.packed, ps.cs, static_cast<cplx<float>*>(fw));
