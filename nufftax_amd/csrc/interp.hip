@@ -98,9 +98,7 @@ hipError_t interp_impl(const GridOpArgs& ga, const void* fw, void* c, hipStream_
     } else {
       const char* gw = std::getenv("NUFFTX_GLOBAL_WAVE");
       if (!(gw && gw[0] == '0')) {
-        // one wave per point (four per block)
-        const unsigned nblk = (unsigned)((ps.M + 3) / 4);
-        hipLaunchKernelGGL((k_gather_global_wave<T, CT, D, NS>), dim3(nblk, (unsigned)ga.n_trans), dim3(256), 0, s, a,
+        hipLaunchKernelGGL((k_gather_global_wave<T, CT, D, NS>), wave_grid(ps.M, ga.n_trans), dim3(256), 0, s, a,
                            static_cast<const cplx<T>*>(fw), static_cast<cplx<T>*>(c));
       } else {
         const unsigned nblk = (unsigned)((ps.M + 255) / 256);

@@ -85,6 +85,16 @@ __device__ __forceinline__ int wrap_near(int g, int n) {
   return g;
 }
 
+// One wave per point, four per block: the wave's point.  A launch has fewer than 2^32 threads in x, so more than 2^25
+// points fold into z (wave_grid).
+__device__ __forceinline__ int64_t wave_slot() {
+  return (((int64_t)blockIdx.z * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
+}
+inline dim3 wave_grid(int64_t M, int64_t n_trans) {
+  const int64_t blocks = (M + 3) / 4, x = std::min<int64_t>(blocks, (int64_t)1 << 23);
+  return dim3((unsigned)x, (unsigned)n_trans, (unsigned)((blocks + x - 1) / x));
+}
+
 template <int D>
 __device__ __forceinline__ void tile_origin(const int4& sd, const int (&bs)[3], const int (&nb)[3], int half,
                                             int (&org)[3]) {
@@ -685,8 +695,8 @@ __global__ void __launch_bounds__(256) k_spread_global_wave(SIArgs<T> a, const c
   constexpr int R = 64 / RL;  // support rows per instruction
   static_assert((D == 2 || D == 3) && D * NS <= 64 && R >= 1, "one wave holds the D NS weights and a support row");
   const int lane = (int)(threadIdx.x & 63);
-  const int64_t j = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;  // sorted slot of this wave's point
-  if (j >= a.M) return;                                                     // uniform over the wave
+  const int64_t j = wave_slot();  // sorted slot of this wave's point
+  if (j >= a.M) return;           // uniform over the wave
   const int tr = blockIdx.y;
   const int p = a.perm[j];
   if ((unsigned)p >= (unsigned)a.M) return;
@@ -1133,8 +1143,8 @@ __global__ void __launch_bounds__(256) k_gather_global_wave(SIArgs<T> a, const c
   constexpr int NY = (NS + R - 1) / R;  // instructions per slice
   static_assert((D == 2 || D == 3) && D * NS <= 64, "one wave holds the D NS weights");
   const int lane = (int)(threadIdx.x & 63);
-  const int64_t j = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;  // sorted slot of this wave's point
-  if (j >= a.M) return;                                                     // uniform over the wave
+  const int64_t j = wave_slot();  // sorted slot of this wave's point
+  if (j >= a.M) return;           // uniform over the wave
   const int tr = blockIdx.y;
   const int p = a.perm[j];
   if ((unsigned)p >= (unsigned)a.M) return;

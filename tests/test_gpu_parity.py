@@ -1084,6 +1084,28 @@ def test_interp64_vs_oracle(rng, ns, nfs, M):
         assert R.rel_l2(_np(out)[t], R.interp([R.wrap_pi(x) for x in coords], fw[t], kp)) < 1e-12
 
 
+def test_interp64_more_points_than_waves_in_x():
+    """One wave per point at 2^26 + 77 points (a launch has fewer than 2^32 threads in x): sampled points and the last ones
+    against the oracle."""
+    from nufftax_amd._plan import F64, Plan
+
+    M, nfs, ns = 2**26 + 77, (32, 30, 36), 14
+    kp = R.compute_kernel_params(1e-12)
+    assert kp.nspread == ns
+    g = torch.Generator(device=DEV)
+    g.manual_seed(9)
+    xs = [(torch.rand(M, generator=g, device=DEV, dtype=torch.float64) * 2 - 1) * np.pi for _ in nfs]
+    fw = torch.randn(tuple(reversed(nfs)), generator=g, device=DEV, dtype=torch.complex128)
+    plan = Plan.grid_op(3, nfs, ns, kp.beta, kp.c, 1, F64, torch.device(DEV, 0))
+    plan.setpts(xs)
+    out = torch.full((M,), float("nan"), dtype=torch.complex128, device=DEV)
+    plan.interp(fw, out)
+    at = torch.cat([torch.randint(M, (300,), generator=g, device=DEV), torch.arange(M - 100, M, device=DEV)])
+    want = R.interp([R.wrap_pi(_np(x[at])) for x in xs], _np(fw), kp)
+    assert R.rel_l2(_np(out[at]), want) < 1e-12
+    assert bool(torch.isfinite(torch.view_as_real(out)).all())
+
+
 # ------------------------------------------------------------------ 3D FP32 interpolation on the matrix cores
 
 
