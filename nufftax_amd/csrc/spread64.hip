@@ -516,18 +516,21 @@ int64_t runs64(const Geometry& g) {  // most runs around a region
 }  // namespace
 
 // Whether M points on a geometry are spread by regions: 3D FP64, supports that fit the grid, runs and weights
-// that fit their bounds, and where it is the faster one (whole type-1 calls, uniform points, against the atomic
-// kernels): the atomic kernels' work grows with ns^3, the regions' little with ns, so from ns = 12 on at every size
-// measured (2048 points on 32^3: 243 -> 87 us; 500k clustered points on 128^3, ns = 14: 4635 -> 1040 us); at ns = 8
-// and 10 from 100 regions on (50k points, ns = 8: 48^3 grid, 54 regions, 133 -> 172 us, 128^3, 1024 regions, 439 ->
-// 259 us; 30k points, ns = 10: 40^3, 45 regions, 132 -> 168 us, 64^3, 128 regions, 296 -> 183 us); not below (50k
-// points on 128^3: ns = 6 299 -> 249 us uniform but 194 -> 228 us clustered, and 1M points 457 -> 826 us).
+// that fit their bounds, and where it is the faster one (whole type-1 calls, against the atomic kernels): the atomic
+// kernels' work grows with ns^3, the regions' little with ns, so from ns = 12 on at every size measured (2048 points on
+// 32^3: 126 -> 86 us; 500k clustered points on 128^3, ns = 14: 4635 -> 1040 us); at ns = 10 from 100 regions on (20k uniform
+// points: 32^3 grid, 16 regions, 96 -> 124 us, 64^3, 128 regions, 283 -> 149 us).  At ns = 8 the atomic kernels are slow where
+// points crowd the tiles' cells, so it depends on the points: 400 regions and more 1.0 .. 3.5x (but 0.85x for 2100
+// clustered points on 96^3); 100 .. 400 regions clustered points from 20k on 1.2 .. 2.0x, uniform ones 0.76 .. 1.1x (64^3:
+// 20k points 107 -> 135 us uniform, 221 -> 132 clustered), fewer points 0.74 .. 1.17x, so from 16384 points on.  Not below
+// (50k points on 128^3: ns = 6 299 -> 249 us uniform but 194 -> 228 us clustered, and 1M points 457 -> 826 us).
 bool spread64_applicable(const Geometry& g, int prec, int64_t M, int64_t n_trans) {
   if (g.dim != 3 || prec != kF64 || g.ns < 8 || M < kSpread64MinPoints) return false;
   for (int d = 0; d < 3; ++d)
     if (g.nf[d] < g.ns) return false;
   const Sizes64 z = sizes64(g, M);
   if (g.ns < 12 && z.regions < 100) return false;
+  if (g.ns == 8 && z.regions < 400 && M < 16384) return false;
   return z.regions < INT32_MAX && runs64(g) <= kRunsMax &&
          M * 3 * g.ns * (int64_t)sizeof(double) <= kTabMaxBytes && spread64_bytes(g, M, n_trans) <= kMaxBytes64 &&
          z.tasks <= (INT32_MAX - kBlocks64) / n_trans;  // a task number per transform, and one past the last per block

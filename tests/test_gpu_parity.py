@@ -1021,6 +1021,22 @@ def test_spread64_regions_non_finite(rng):
     assert R.rel_l2(got[1][~touched], ref[1][~touched]) < 1e-13
 
 
+@pytest.mark.parametrize("nfs,M", [((70, 64, 60), 16384), ((96, 100, 90), 2048)])
+def test_spread64_regions_at_ns_8(rng, nfs, M):
+    """ns = 8 on both sides of its rule (fewer regions and many points, many regions and few points): FP64 accumulation in
+    another order than the oracle's, 1e-13 of the grid's norm."""
+    from nufftax_amd._plan import F64, Plan
+
+    kp = R.compute_kernel_params(1e-7)
+    coords = [rng.uniform(-np.pi, np.pi, M) for _ in nfs]
+    c = rng.standard_normal((1, M)) + 1j * rng.standard_normal((1, M))
+    plan = Plan.grid_op(3, nfs, kp.nspread, kp.beta, kp.c, 1, F64, torch.device(DEV, 0))
+    plan.setpts([_t(x) for x in coords])
+    fw = _t(np.full((1,) + tuple(reversed(nfs)), np.nan + 0j))
+    plan.spread(_t(c), fw)
+    assert R.rel_l2(_np(fw)[0], R.spread([R.wrap_pi(x) for x in coords], c[0], nfs, kp)) < 1e-13
+
+
 # ------------------------------------------------------------------ mixed-radix FFT + deconvolution passes
 
 

@@ -472,3 +472,15 @@ def test_fp64_region_spread_is_bounded_in_points_and_transforms():
         assert M * (24 * ns + 16 + 24 * n_trans) <= held(M, n_trans) <= 4 << 30
     for M, n_trans in ((2_000_000, 75), (2_000_000, 1000), (6_300_000, 342), (6_500_000, 1), (2**31 - 2, 1), (2**31 - 2, 65535)):
         assert held(M, n_trans) == 0
+
+
+def test_fp64_region_spread_at_ns_8_needs_regions_or_points():
+    """At ns = 8 small point sets on 64^3 grids (128 regions), where the region spread was the slower one for every
+    distribution measured, keep the atomic kernels and need no buffers for it."""
+    from nufftax_amd import _lib
+    from nufftax_amd._plan import F64
+
+    assert R.compute_kernel_params(1e-7).nspread == 8
+    held = lambda M, n: _lib.workspace_bytes(1, (n, n, n), 1, 1e-7, F64, M)  # noqa: E731  (grids below 700k cells: no FFT passes)
+    assert held(8000, 32) == 0 and held(16383, 32) == 0 and held(16384, 32) > 0
+    assert held(8000, 48) > held(100, 48)  # 96^3 cells, 432 regions
