@@ -22,7 +22,7 @@ constexpr int kSpread1dCells = 4096;   // 64 KB of accumulators
 constexpr int kInterp1dCells = 4096;   // 32 KB (FP32) or 64 KB (FP64) of grid
 constexpr int kThreads1d = 512;
 constexpr int kPpt1d = 4;              // points per thread and step
-constexpr int kBlocks1d = 512;         // blocks that share a transform's points at most
+constexpr int kBlocks1d = 512;         // blocks of a launch aimed at where there are more points than a step of each
 
 template <typename T>
 struct Args1d {
@@ -180,17 +180,19 @@ Args1d<T> args1d(const GridOpArgs& ga, int per_block) {
   return a;
 }
 
-// points per block: one step of every thread at least, at most kBlocks1d blocks
-int points_per_block(int64_t M, int step) {
-  const int64_t p = (M + kBlocks1d - 1) / kBlocks1d;
+// points per block: one step of every thread at least, at most `blocks` blocks
+int points_per_block(int64_t M, int step, int64_t blocks) {
+  const int64_t p = (M + blocks - 1) / blocks;
   return (int)((std::max<int64_t>(p, step) + kThreads1d - 1) / kThreads1d * kThreads1d);
 }
 
 template <typename T, typename CT>
 hipError_t spread1d_run(const GridOpArgs& ga, const void* c, void* fw, hipStream_t s) {
   const int64_t M = ga.ps->M;
-  // up to one block's worth of points: the block stores the grid (no clear, no atomics)
-  const int per = points_per_block(M, kThreads1d * kPpt1d);
+  // Up to one block's worth of points: the block stores the grid (no clear, no atomics).  All transforms together have
+  // kBlocks1d blocks, two per CU: each adds a whole grid to memory with atomics, which 512 blocks for each of several
+  // transforms spent most of their time on (8 FP64 transforms of 1M points, 4096 cells: 455 us, now 251; sorted 303).
+  const int per = points_per_block(M, kThreads1d * kPpt1d, std::max<int64_t>(1, kBlocks1d / ga.n_trans));
   const unsigned nb = (unsigned)((M + per - 1) / per);
   const Args1d<T> a = args1d<T>(ga, per);
   const int store = nb == 1 && ga.zero_out ? 1 : 0;
@@ -214,7 +216,7 @@ hipError_t interp1d_run(const GridOpArgs& ga, const void* fw, void* c, hipStream
   const int64_t M = ga.ps->M;
   const bool lds = ga.g->nf[0] <= kInterp1dCells;
   // (a block that reads the grid from memory gains nothing from more points)
-  const int per = lds ? points_per_block(M, kThreads1d) : kThreads1d;
+  const int per = lds ? points_per_block(M, kThreads1d, kBlocks1d) : kThreads1d;
   const unsigned nb = (unsigned)((M + per - 1) / per);
   const Args1d<T> a = args1d<T>(ga, per);
   const size_t bytes = lds ? (size_t)a.nf * sizeof(cplx<T>) : 0;

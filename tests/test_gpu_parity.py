@@ -1287,6 +1287,25 @@ def test_direct1d_vs_oracle(rng, prec, ns, nf, M):
     assert R.rel_l2(_np(fw), want + g) < tol
 
 
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+def test_direct1d_many_transforms_share_the_blocks(rng, prec):
+    """64 transforms: 8 blocks each, several steps per block.  Tolerances of test_direct1d_vs_oracle."""
+    from nufftax_amd._plan import F32, F64, Plan
+
+    nf, ns, M, nt = 4096, 8, 20000, 64
+    rdt, cdt, pr, tol = (np.float32, np.complex64, F32, 2e-6) if prec == "f32" else (np.float64, np.complex128, F64, 1e-12)
+    kp = R.compute_kernel_params(1e-7)
+    x = rng.uniform(-np.pi, np.pi, M).astype(rdt)
+    c = (rng.standard_normal((nt, M)) + 1j * rng.standard_normal((nt, M))).astype(cdt)
+    plan = Plan.grid_op(1, (nf,), ns, kp.beta, kp.c, nt, pr, torch.device(DEV, 0))
+    plan.setpts([_t(x)])
+    fw = torch.empty((nt, nf), dtype=torch.complex64 if prec == "f32" else torch.complex128, device=DEV)
+    plan.spread(_t(c), fw)
+    for t in (0, 1, 37, 63):
+        want = R.spread([R.wrap_pi(x.astype(np.float64))], c[t].astype(np.complex128), (nf,), kp)
+        assert R.rel_l2(_np(fw)[t], want) < tol
+
+
 def test_direct1d_sorts_when_asked(rng):
     """A 1D plan that has not needed its sort makes it for the sort state and for coordinate gradients."""
     from nufftax_amd._plan import F32, Plan
