@@ -41,6 +41,7 @@ struct PointSet {
   bool coord_f64 = false;
   // sort state (1D point sets are sorted on their first use that needs it, see direct1d.hip)
   bool sorted = false;
+  unsigned long long sort_capture = 0;  // stream capture that holds their sort, if that is the only one made
   int NB = 0;        // sort chunks (rows of the histogram matrix)
   int CH = 0;        // points per chunk
   int maxsub = 0;    // max points per subproblem

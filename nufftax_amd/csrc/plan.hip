@@ -524,22 +524,29 @@ int sort_points(nufftx_plan p, PointSet& ps, const Geometry& g, bool interp, boo
 }
 
 // Sorts a point set of setpts that has not been sorted yet (1D: direct1d.hip needs no sort).  A sort that is captured into a
-// graph runs with its replays only, so the points stay unsorted for every other call.
+// graph runs with its replays only: it serves the later calls of that capture, and the points stay unsorted for every other.
 int need_sorted(nufftx_plan p, bool inner, bool reserve_only = false) {
   PointSet& ps = inner ? p->pt : p->ps;
   if (ps.sorted) return NUFFTX_OK;
-  const int r = sort_points(p, ps, inner ? p->gi : p->g, inner || p->type != 1, !inner && p->type != 2, reserve_only);
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (ps.sorted && (inner ? p->gi : p->g).dim == 1 && hipStreamIsCapturing(p->stream, &st) == hipSuccess &&
-      st != hipStreamCaptureStatusNone)
+  unsigned long long id = 0;
+  const bool capturing = (inner ? p->gi : p->g).dim == 1 && hipStreamGetCaptureInfo(p->stream, &st, &id) == hipSuccess &&
+                         st == hipStreamCaptureStatusActive;
+  if (capturing && id != 0 && ps.sort_capture == id) return NUFFTX_OK;
+  const int r = sort_points(p, ps, inner ? p->gi : p->g, inner || p->type != 1, !inner && p->type != 2, reserve_only);
+  if (ps.sorted && capturing) {
     ps.sorted = false;
+    ps.sort_capture = id;
+  }
   return r;
 }
 
 // setpts: sort now, unless neither the forward use nor (1D) anything else needs it yet
 int set_points(nufftx_plan p, bool inner) {
   const Geometry& g = inner ? p->gi : p->g;
-  (inner ? p->pt : p->ps).sorted = false;
+  PointSet& ps = inner ? p->pt : p->ps;
+  ps.sorted = false;
+  ps.sort_capture = 0;
   const bool spreads = !inner && (p->type == 1 || p->type == 3);
   // the buffers of a later sort are sized here, so that a captured call allocates nothing
   const bool later = g.dim == 1 && interp1d_direct(g) && (!spreads || spread1d_direct(g));

@@ -1122,6 +1122,60 @@ def test_interp64_more_points_than_waves_in_x():
     assert bool(torch.isfinite(torch.view_as_real(out)).all())
 
 
+def test_captured_1d_sort_is_made_once(rng):
+    """setpts and execute captured together hold the sort once: as many graph nodes as setpts alone and execute alone (type 1
+    on a grid that is spread from sorted points).  The graph's replays and a later eager call agree with another plan."""
+    import ctypes
+
+    from nufftax_amd import _lib
+    from nufftax_amd._plan import F32, Plan
+
+    L = _lib.lib()
+    M, nm, dev = 3000, 5000, torch.device(DEV, 0)
+    x = _t(rng.uniform(-np.pi, np.pi, M).astype(np.float32))
+    c = _t((rng.standard_normal(M) + 1j * rng.standard_normal(M)).astype(np.complex64))
+    out, want = torch.empty(nm, dtype=torch.complex64, device=DEV), torch.empty(nm, dtype=torch.complex64, device=DEV)
+    other = Plan.transform(1, 1, (nm,), 1, 1e-6, 1, 2.0, F32, 0, dev)
+    other.setpts([x])
+    other.execute(c, want)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        plan = Plan.transform(1, 1, (nm,), 1, 1e-6, 1, 2.0, F32, 0, dev)
+        plan.setpts([x])
+        plan.execute(c, out)
+        torch.cuda.synchronize()
+        handle = ctypes.c_void_p(side.cuda_stream)
+
+        def nodes(*calls):
+            graph, n = ctypes.c_void_p(), ctypes.c_size_t()
+            assert L.hipStreamBeginCapture(handle, 1) == 0
+            for call in calls:
+                call()
+            assert L.hipStreamEndCapture(handle, ctypes.byref(graph)) == 0
+            assert L.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+            assert L.hipGraphDestroy(graph) == 0
+            return n.value
+
+        setpts, execute = lambda: plan.setpts([x]), lambda: plan.execute(c, out)
+        setpts()
+        alone = nodes(execute)
+        assert nodes(setpts, execute) == nodes(setpts) + alone
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            setpts()
+            execute()
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert R.rel_l2(_np(out), _np(want)) < 2e-6
+        out.zero_()
+        execute()
+        torch.cuda.synchronize()
+    assert R.rel_l2(_np(out), _np(want)) < 2e-6
+
+
 # ------------------------------------------------------------------ 3D FP32 interpolation on the matrix cores
 
 
