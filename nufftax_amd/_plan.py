@@ -123,12 +123,13 @@ class Plan:
         xs = [t.data_ptr() for t in coords] + [None] * (3 - len(coords))
         ss = [t.data_ptr() for t in targets] + [None] * (3 - len(targets))
         self._pts_key = None
+        # kept from here on: the plan holds the pointers also where the points are set and the execute fails
+        self._pts_refs = (coords, targets)
+        self.M, self.N = M, N
         check(
             lib().nufftx_run(self.h, _stream_handle(self.device), M, *xs, N, *ss, c.data_ptr(), f.data_ptr(), isign),
             "nufftx_run",
         )
-        self._pts_refs = (coords, targets)
-        self.M, self.N = M, N
 
     def execute(self, c, f, isign=None):
         self._sync_stream()

@@ -484,3 +484,22 @@ def test_fp64_region_spread_at_ns_8_needs_regions_or_points():
     held = lambda M, n: _lib.workspace_bytes(1, (n, n, n), 1, 1e-7, F64, M)  # noqa: E731  (grids below 700k cells: no FFT passes)
     assert held(8000, 32) == 0 and held(16383, 32) == 0 and held(16384, 32) > 0
     assert held(8000, 48) > held(100, 48)  # 96^3 cells, 432 regions
+
+
+def test_run_keeps_the_points_of_a_failed_execute(monkeypatch):
+    """Plan.run sets points and executes in one call.  If only the execute fails the library still holds the points' pointers,
+    so the plan keeps their tensors (and their number, which sort_state reads)."""
+    import types
+
+    import torch
+
+    from nufftax_amd import _plan
+
+    plan = _plan.Plan(ctypes.c_void_p(), 1, 1, 0, 1, torch.device("cpu"))
+    fake = types.SimpleNamespace(nufftx_run=lambda *a: 1, nufftx_last_error=lambda: b"execute failed")
+    monkeypatch.setattr(_plan, "lib", lambda: fake)
+    monkeypatch.setattr(_plan, "_stream_handle", lambda device: 0)
+    x, c, f = torch.zeros(5), torch.zeros(5, dtype=torch.complex64), torch.zeros(8, dtype=torch.complex64)
+    with pytest.raises(Exception):
+        plan.run([x], (), c, f, 1)
+    assert plan._pts_refs[0][0] is x and plan.M == 5
