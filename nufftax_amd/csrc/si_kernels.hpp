@@ -154,8 +154,7 @@ __device__ __forceinline__ void load_tile(const SIArgs<T>& a, const cplx<T>* __r
   for (int cell = threadIdx.x; cell < n; cell += 4 * step) {
     cplx<T> v[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u, w.next())
-      if (cell + u * step < n) v[u] = fT[w.at(org, a.nf)];
+    for (int u = 0; u < 4; ++u, w.next()) v[u] = fT[w.at(org, a.nf)];  // (past the tile: some cell of the grid)
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       if (cell + u * step < n) tile[cell + u * step] = v[u];

@@ -503,3 +503,13 @@ def test_run_keeps_the_points_of_a_failed_execute(monkeypatch):
     with pytest.raises(Exception):
         plan.run([x], (), c, f, 1)
     assert plan._pts_refs[0][0] is x and plan.M == 5
+
+
+def test_fp64_tiled_gathers_keep_their_cells_in_registers():
+    """The four cells that a thread of a tiled gather has in flight while it loads its tile are registers, not scratch memory
+    (FP64 values: every 2D width, and the 3D widths whose points fit the registers)."""
+    kernels = _kernel_metadata()
+    for dim, widths in ((2, range(2, 17, 2)), (3, (2, 4))):
+        for ns in widths:
+            found = [k for n, k in kernels.items() if f"k_gather_tiledIddLi{dim}ELi{ns}ELb0ELb0E" in n]
+            assert found and all(k[".private_segment_fixed_size"] == 0 for k in found), (dim, ns)
