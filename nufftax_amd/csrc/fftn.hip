@@ -516,6 +516,9 @@ bool fftn_applicable(const DeconvArgs& a) {
     if (name[0])
       if (const char* e = std::getenv(name))
         if (e[0] == '0') return false;
+  // 1D FP32 beyond 8M cells stays with rocFFT: both halves of the split have some 3000 points there, whose sequences leave
+  // runs of 8 and 16 bytes (type 1 of 500 points: 8M cells 183 us, rocFFT 195; 9M 253, 220; 12M 328, 276.  FP64 12M 520, 555)
+  if (a.dim == 1 && a.prec == kF32 && a.nf[0] > 8000000) return false;
   for (int d = 0; d < a.dim; ++d) {
     if (a.nf[d] < 2 || a.nm[d] > a.nf[d]) return false;
     if (!axis_fits(a.nf[d], a.prec) && (a.dim > 1 || split_length(a.nf[d], a.prec) == 0)) return false;

@@ -513,3 +513,12 @@ def test_fp64_tiled_gathers_keep_their_cells_in_registers():
         for ns in widths:
             found = [k for n, k in kernels.items() if f"k_gather_tiledIddLi{dim}ELi{ns}ELb0ELb0E" in n]
             assert found and all(k[".private_segment_fixed_size"] == 0 for k in found), (dim, ns)
+
+
+def test_fft_passes_of_long_1d_axes():
+    """1D FP32 grids of more than 8M cells keep rocFFT, whose two passes are the faster ones there: no intermediate."""
+    from nufftax_amd import _lib
+    from nufftax_amd._plan import F32
+
+    held = lambda n: _lib.workspace_bytes(1, (n,), 1, 1e-4, F32, 1000)  # noqa: E731
+    assert held(3_000_000) == 6_000_000 * 8 and held(6_000_000) == 0
