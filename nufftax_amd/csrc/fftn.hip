@@ -292,14 +292,15 @@ bool factorise(int n, int most, std::vector<int>& best, std::vector<int>& cur, i
   return any;
 }
 
-// Radices above 10 take the registers of a third of the waves: FP32 axes use them where they leave two passes
-// (192-point axis of 180 x 192 x 200: 27 us, 34 without), or three on a long axis (1600: 35, 42), not to save the
-// fourth pass of a short one (375: 13, 9); FP64 axes never (128^3: 75 us, 48 without).
-std::vector<int> radices_of(int n, int prec) {
+// Radices above 10 take the registers of some of the waves: FP32 axes use them where they leave two passes in 3D (type 1 of
+// 500 points on 160^3: 88 us, 95 without; not in 2D, whose passes are short of waves: 4 transforms on 240 x 240 42.5,
+// 39.4), or three on a long axis (1440 x 1440: 73.5, 77.1), not to save the fourth pass of a short one (type 2 on
+// 375 x 375: 39.2, 37.0); FP64 axes never (2400 x 2400: 140, 129).
+std::vector<int> radices_of(int n, int prec, int dim) {
   std::vector<int> best, cur;
   for (int most = 1; most <= kMaxPasses && best.empty() && n > 1; ++most) {
     factorise(n, most, best, cur, 3);  // up to 10
-    if (best.empty() && prec == kF32 && (most == 2 || (most == 3 && n > 1024))) factorise(n, most, best, cur, 0);
+    if (best.empty() && prec == kF32 && ((most == 2 && dim == 3) || (most == 3 && n > 1024))) factorise(n, most, best, cur, 0);
   }
   // odd radices first: the first pass writes with a stride of its radix
   std::stable_partition(best.begin(), best.end(), [](int r) { return r % 2 != 0; });
@@ -307,9 +308,9 @@ std::vector<int> radices_of(int n, int prec) {
 }
 
 // Whether one pass transforms an axis of n points: its threads and its LDS (twiddles and one sequence) fit a block.
-bool axis_fits(int n, int prec) {
+bool axis_fits(int n, int prec, int dim) {
   if (n < 2 || n > kMaxLen) return false;
-  const std::vector<int> r = radices_of(n, prec);
+  const std::vector<int> r = radices_of(n, prec, dim);
   if (r.empty()) return false;
   const int lo = *std::min_element(r.begin(), r.end()), hi = *std::max_element(r.begin(), r.end());
   const int real_bytes = prec == kF32 ? 4 : 8;
@@ -320,7 +321,7 @@ bool axis_fits(int n, int prec) {
 // N = Na Nb, as near as can be, with axes that fit; 0 if there is none
 int split_length(int n, int prec) {
   for (int a = (int)std::sqrt((double)n) + 1; a >= 2; --a)
-    if (n % a == 0 && axis_fits(a, prec) && axis_fits(n / a, prec)) return a;
+    if (n % a == 0 && axis_fits(a, prec, 1) && axis_fits(n / a, prec, 1)) return a;
   return 0;
 }
 
@@ -521,21 +522,21 @@ bool fftn_applicable(const DeconvArgs& a) {
   if (a.dim == 1 && a.prec == kF32 && a.nf[0] > 8000000) return false;
   for (int d = 0; d < a.dim; ++d) {
     if (a.nf[d] < 2 || a.nm[d] > a.nf[d]) return false;
-    if (!axis_fits(a.nf[d], a.prec) && (a.dim > 1 || split_length(a.nf[d], a.prec) == 0)) return false;
+    if (!axis_fits(a.nf[d], a.prec, a.dim) && (a.dim > 1 || split_length(a.nf[d], a.prec) == 0)) return false;
   }
   return true;
 }
 
 int64_t fftn_mid_bytes(const DeconvArgs& a) {
   const int64_t n0 = a.nm[0], f0 = a.nf[0], f1 = a.nf[1], f2 = a.nf[2];
-  const int64_t cells = a.dim == 1 ? (axis_fits(a.nf[0], a.prec) ? 0 : f0) : a.dim == 2 ? f1 * n0 : f2 * f1 * n0;
+  const int64_t cells = a.dim == 1 ? (axis_fits(a.nf[0], a.prec, 1) ? 0 : f0) : a.dim == 2 ? f1 * n0 : f2 * f1 * n0;
   return cells * a.n_trans * (a.prec == kF32 ? 8 : 16);
 }
 
 hipError_t fftn_plan_init(FftnPlan& fp, const DeconvArgs& a) {
   hipError_t e;
   int len[3] = {a.nf[0], a.nf[1], a.nf[2]}, n = a.dim;
-  if (a.dim == 1 && !axis_fits(a.nf[0], a.prec)) {
+  if (a.dim == 1 && !axis_fits(a.nf[0], a.prec, 1)) {
     fp.split = split_length(a.nf[0], a.prec);
     len[0] = fp.split;
     len[1] = a.nf[0] / fp.split;
@@ -543,7 +544,7 @@ hipError_t fftn_plan_init(FftnPlan& fp, const DeconvArgs& a) {
   }
   for (int d = 0; d < n; ++d) {
     fp.axis[d].n = len[d];
-    fp.axis[d].radix = radices_of(len[d], a.prec);
+    fp.axis[d].radix = radices_of(len[d], a.prec, a.dim);
     e = a.prec == kF32 ? twiddle_table<float>(fp.axis[d].tw, len[d]) : twiddle_table<double>(fp.axis[d].tw, len[d]);
     if (e != hipSuccess) return e;
   }
