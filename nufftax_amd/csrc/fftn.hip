@@ -7,11 +7,12 @@
 // already (type 1: x, y, z), so nothing is done for padding: a 3D type 2 with n of 2 n bins per axis
 // moves (1/8 + 1/4) + (1/4 + 1/2) + (1/2 + 1) of the grid, where a library FFT after a padding pass moves 1/8 + 1 and
 // 6, its strided axes at a fraction of the memory's rate (540^3 FP64, 2.5 GB, from 270^3 modes: rocFFT and the
-// padding pass 5400 us; these passes 1800).  The x pass, the largest, reads and writes whole rows;
-// y and z passes take S neighbouring x at once (runs of 128 bytes) and keep the order of the axes.  (An earlier
-// form, contiguous reads and transposed writes on every axis, took 3440 us: its last pass wrote 64-byte runs
-// over 540 planes.)  Axes longer than kMaxLen (1D) are split N = Na Nb (four-step, Bailey 1990): length-Na
-// transforms over every Nb-th value, times exp(-2 pi i b n / N), then length-Nb ones.
+// padding pass 5400 us; these passes 1600: x, y and z 3.8, 1.9 and 0.95 GB at 4.7, 3.9 and 3.3 TB/s, where a large copy
+// reaches 4.8).  The x pass, the largest, reads and writes whole rows; y and z passes take S neighbouring x at once (runs
+// of 128 bytes) and keep the order of the axes.  (An earlier form, contiguous reads and transposed writes on every axis,
+// took 3440 us: its last pass wrote 64-byte runs over 540 planes.)  Axes longer than
+// kMaxLen (1D) are split N = Na Nb (four-step, Bailey 1990): length-Na transforms over every Nb-th value, times
+// exp(-2 pi i b n / N), then length-Nb ones.
 //
 // A sequence of N = R_1 R_2 .. points is transformed by Stockham passes (fft2d.hip describes the recurrence) of
 // radix 2 .. 16, each thread taking one R-point column in registers (fft_dft.hpp), T = max N / R threads

@@ -24,9 +24,9 @@ bool interp_by_wave(const Geometry& g, int64_t M) {
 }
 
 // The 3D matrix-core gather: ns = 8, bins of whole 8 x 8 x 4 sub-bins (at most 16).  Whole type-2 calls, 32^3 .. 128^3
-// modes, uniform and clustered, 0.003 .. 0.8 points per cell: 1.08 .. 1.31x faster than the thread-per-point gather (8M
-// clustered points, 128^3: 1531 -> 1326 us).  At ns = 6 that one stays (0.79 .. 0.98x otherwise): its work falls with
-// ns^3, that of the windows hardly.
+// modes, uniform and clustered, 0.003 .. 0.8 points per cell: 1.12 .. 1.19x faster than the thread-per-point gather (8M
+// clustered points, 128^3: 1540 -> 1372 us; 20k points, 32^3: 70 -> 61).  At ns = 6 that one stays
+// (0.79 .. 0.98x otherwise): its work falls with ns^3, that of the windows hardly.
 bool gather3_applicable(const Geometry& g) {
   if (g.dim != 3 || g.ns != 8) return false;
   if (g.bs[0] % kW3SB || g.bs[1] % kW3SB || g.bs[2] % kW3SBZ) return false;

@@ -5,16 +5,18 @@
 // so for 16 points the x sums of one z slice and part are one matrix product G = F Bx.  F and wx are split into
 // two fp16 parts (hi + lo: 22 bits and more, scaled to the top of fp16's range, as in the spread), and the K = 32 of
 // v_mfma_f32_16x16x32_f16 holds the 16 x twice, [F_lo | F_hi] against [B_lo ; B_lo] and then [B_hi ; B_hi]: all four
-// products in two instructions, nothing left out but the roundings of lo, the small ones summed first.  The tile is staged in LDS already split,
-// as four fp16 planes (re and im, hi and lo: 8 bytes a cell, as FP32), so that a lane reads 8 cells of one plane
+// products in two instructions, nothing left out but the roundings of lo, the small ones summed first.  The tile is staged in LDS
+// already split, as four fp16 planes (re and im, hi and lo: 8 bytes a cell, as FP32), so that a lane reads 8 cells of one plane
 // with one 16-byte read, its operand; a window is read once per sub-bin that a wave visits, into (4 + ns) * 8
 // registers.  A group then costs two MFMAs and 5 FMAs per slice and part.  (Windows read from the grid by each wave,
 // 64 rows a load: 1937 us where the thread-per-point gather takes 1170; 8M points.)
 //
 // What bounds the thread-per-point gather (k_gather_wide) is its LDS: 8 ns^3 bytes and a quarter per point, at scattered
 // rows (8M clustered points, ns = 8, 128^3 modes: 41 GB, 520 us at the LDS's rate, 1170 measured).  Here a point's cells
-// are shared by its group, and the vector instructions bound it: about 400 a group beside its 48 MFMAs (510 us at full
-// issue); 950 us measured with two blocks per CU (78 KB of LDS, 187 registers).
+// are shared by its group.  1031 us measured for those points, two blocks per CU (78 KB of LDS, 191 registers); counters:
+// vector units 49% busy, matrix cores 17%, LDS 6%, and 3.9 GB fetched, most of it lines of 128 bytes for coordinates
+// read through the sort's permutation (96 MB of them): memory and arithmetic take about 0.8 and 0.7 of the time, in part
+// one after the other.
 //
 // Block = one subproblem (points of one bin, 1024 at a time), 4 waves:
 //   1. order: every point's words (support start in the tile, fraction) into LDS, and its place in sub-bin order

@@ -350,9 +350,8 @@ __global__ void __launch_bounds__(kWinThreads) k_spread_win2d(SIArgs<float> a, i
 // hi = fp16(v) and lo = fp16(v - hi), and each window accumulates
 //   A_hi B_hi + A_lo B_hi + A_hi B_lo          (three MFMAs per part, FP32 accumulation),
 // which leaves out A_lo B_lo and the rounding of lo: at most 2^-22 |A| |B| per term.  Both
-// operands are scaled to the top of fp16's range, so that lo parts stay normal numbers (the
-// matrix cores flush fp16 subnormal inputs: with B = wx in [0, 1] the lo parts of weights
-// below 2^-3 were lost, a 5e-6 relative error on the 2D radial workload):
+// operands are scaled to the top of fp16's range, so that lo parts stay normal numbers
+// (subnormal ones, which the matrix cores take as they are, resolve 2^-24 only):
 // A = ldexp(c, 15 - e) wy with 2^e above the subproblem's max |re c|, |im c| (|A| < 2^15) and
 // B = 2^14 wx (B < 2^15); lo is then normal down to |A|, B = 2^-3, i.e. relative to the
 // largest operand 2^-18, and the terms lost below that are under 2^-29 of it.

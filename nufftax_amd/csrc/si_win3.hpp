@@ -14,8 +14,8 @@
 // sub-bins (at most 16 per bin); the 3D sort's bins of 16 x 8 x 8 or 16 x 16 x 8 cells are.
 //
 // Block = one subproblem (<= 4096 points of one bin), 8 waves:
-//   1. order: as in the 2D kernel (eight points per thread), sub-bins padded to multiples of
-//      32 with zero-strength entries; the block also takes max(|re c|, |im c|) and
+//   1. order: as in the 2D kernel (four or eight points per thread), sub-bins padded to multiples
+//      of 32 with zero-strength entries; the block also takes max(|re c|, |im c|) and
 //      S = sum_j max(|re c_j|, |im c_j|);
 //   2. accumulate: contiguous ranges of groups per wave; per group, the lanes evaluate the
 //      kernel weights of the 32 points into LDS rows (x and y: 17 floats a row, 16 - ns zeros
@@ -31,7 +31,8 @@
 // What bounds it: the flush's global atomics and one block per CU, whose phases do not overlap.  8M clustered points with
 // 128^3 modes in subproblems of 2048: 141M atomics (430 us at the 330 G/s that coalesced FP32 atomics reach), 1331 us.
 // Subproblems of 4096, which the weights' blocks leave room for since the strengths moved into the meta words, flush the
-// dense bins half as often: the whole call 1960 -> 1913 us; taken where the points fill the chip with them (win3_maxsub).
+// dense bins half as often: the whole call 1960 -> 1913 us, the kernel 1288; taken where the points fill the chip with them
+// (win3_maxsub).  Counters of the 8M points: vector units 44% busy, matrix cores 10%, LDS 8%, HBM 0.8 GB.
 // (The counts of passes without points left out of the order phase: 2% slower.)  (Zero window
 // cells skipped in the flush to the tile: 1365.  The tile's words read four at a time in the last flush: 1340.)
 // The per-wave LDS blocks (weight rows, meta, strengths) are whole multiples of 16 bytes: an
